@@ -6,14 +6,22 @@
 // Activations are channel-last on the n^3 index lattice: X[v * C + c], v = (x * ny + y) * nz + z.
 //
 // Forward convolution (k_conv): one persistent block per CU stages the layer's weights in LDS
-// once and walks 4x4x16 bricks of output voxels, computing every output channel of a brick.  The
-// brick's input halo (6x6x18 voxels x CIN channels) is staged in LDS with an 8-byte pad per
-// voxel (conflict-free A-fragment reads; the weight rows carry the same pad), and the next
-// brick's halo is loaded into registers while the current brick computes.  Each wave owns one
-// x-plane of the brick, i.e. four 16-voxel z-rows, and for every tap and 16-channel slice issues
-// one MFMA per (row, 16-output-channel tile): the A operand is 16 voxels x 16 input channels,
-// the B operand 16 input x 16 output channels of the tap's weights, both from LDS.  The epilogue adds the bias, optionally multiplies by silu'(z_saved) and adds a
-// residual, and writes FP32 and/or BF16 (optionally silu-activated) outputs.
+// once and walks a contiguous range of 4x4x16 (or 4x2x16) bricks of output voxels, two at a time,
+// computing every output channel of a brick.  The brick's input halo (6x6x18 voxels x CIN
+// channels) is staged in LDS, its 16-byte pieces permuted so that operand reads are
+// conflict-free, and the next brick's halo is loaded into registers while the current brick
+// computes.  Each wave owns one x-plane of the brick, i.e. four 16-voxel z-rows, and for every tap
+// issues one MFMA per (row, 16-output-channel tile): the A operand is 16 output x 32 (or 16) input
+// channels of the tap's weights, the B operand the input channels of 16 voxels, both from LDS.
+// A lane then holds 4 consecutive output channels of a voxel.  The epilogue adds the bias,
+// optionally multiplies by silu'(z_saved) and adds a residual, and writes FP32 and/or BF16
+// (optionally silu-activated) outputs, 16 bytes a lane.
+//
+// Bound, 32 to 32 channels at 64^3: the first conv of a block 19.2 us (MFMA 1.45e10 flop: 12.4 us
+// at the 1.17 PFLOP/s a large product reaches; 13 us with the MFMAs left out), the second 22.2 us
+// (101 MB with the FP32 residual stream: 20.4 us at the 4.9 TB/s of a copy).  They took 30 and 42
+// us with a weight read ahead of every MFMA pair, 8-byte padded rows (two reads an operand),
+// pair stores and bricks dealt to the XCDs in turn.
 //
 // Data gradient: the same kernel with the weights mirrored in the taps and transposed in the
 // channels.  Weight gradient (k_wgrad): per block and brick, dW[tap][co][ci] += sum over the
@@ -22,6 +30,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include <cmath>
@@ -35,15 +44,10 @@ namespace {
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-
-// 8 consecutive BF16 values from LDS at an 8-byte aligned address, as an MFMA operand
-__device__ __forceinline__ v8bf lds8(const unsigned char* p) {
-    const v4s lo = *(const v4s*)p, hi = *(const v4s*)(p + 8);
-    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 constexpr int BX = 4, BY = 4, BZ = 16;               // output brick of a block
 constexpr int BV = BX * BY * BZ;                     // 256 voxels
@@ -101,67 +105,124 @@ struct ConvArgs {
     int act;              // outb = silu(v) (1) or v (0)
 };
 
-template <int CIN, int COUT>
+// Consecutive work ranges go to one XCD (blocks are dealt round-robin over the 8 XCDs), so that
+// neighbouring bricks meet in that XCD's L2: the rank of block b of nb.
+__device__ __forceinline__ int xcd_rank(int b, int nb) {
+    const int per = nb / 8, rem = nb % 8, xcd = b % 8, slot = b / 8;
+    return xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+}
+
+// One MFMA operand of 16 rows: 32 input channels (16x16x32) or 16 (16x16x16) of them.
+template <bool K32> struct Frag { typedef v8bf T; };
+template <> struct Frag<false> { typedef v4s T; };
+
+__device__ __forceinline__ v4f mma(v8bf a, v8bf b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ v4f mma(v4s a, v4s b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+
+template <int CIN, int COUT, int BY>
 __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
-    constexpr int SV = CIN * 2 + 8;  // LDS bytes per halo voxel and per weight row
-    constexpr int PV = CIN / 4;      // 8-byte pieces per voxel
+    constexpr int HY = BY + 2, HV = HX * HY * HZ;
+    constexpr bool K32 = CIN == 32 && COUT == 32;
+    typedef typename Frag<K32>::T F;
+    constexpr int RB = CIN * 2;             // LDS bytes per halo voxel and per weight row
+    constexpr int PV = CIN / 8;             // 16-byte pieces of one
+    constexpr int NS = K32 ? 1 : CIN / 16;  // MFMA slices of the input channels
     constexpr int NT = COUT / 16;
-    constexpr int NP = HV * PV;      // halo pieces of a brick
-    constexpr int NH = (NP + 255) / 256;
-    __shared__ __align__(16) unsigned char sw[27 * COUT * SV];  // the layer's weights, all bricks
-    __shared__ __align__(16) unsigned char sx[2][HV * SV];      // the two current bricks' halos
+    constexpr int TPR = HZ * PV;            // pieces of a halo row (a z-line of 18 voxels)
+    constexpr int RPI = 216 / TPR;          // halo rows that 216 of a half's threads move at once
+    constexpr int NJ = HX * HY / RPI;
+    static_assert(216 % TPR == 0 && HX * HY % RPI == 0, "halo rows divide among the threads");
+    __shared__ __align__(16) unsigned char sw[27 * COUT * RB];  // the layer's weights, all bricks
+    __shared__ __align__(16) unsigned char sx[2][HV * RB];      // the two current bricks' halos
     const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
     const int nbz = n2 / BZ, nby = n1 / BY;
     // the block's two halves (4 waves each) work on bricks 2 p and 2 p + 1 of pair p
     const int half = threadIdx.x >> 8, ht = threadIdx.x & 255;
-
-    for (int i = threadIdx.x; i < 27 * COUT * PV; i += 512) {
-        const int row = i / PV, p = i - row * PV;
-        *(uint2*)(sw + row * SV + p * 8) = *(const uint2*)(a.w + (long long)row * CIN + p * 4);
-    }
-
-    // the next brick's halo travels in registers while the current brick computes
-    uint2 pre[NH];
-    auto fetch = [&](int bb) {
-        const int bz = bb % nbz, by = (bb / nbz) % nby, bx = bb / (nbz * nby);
-#pragma unroll
-        for (int j = 0; j < NH; ++j) {
-            const int i = ht + j * 256;
-            if (i < NP) {
-                const int v = i / PV, p = i - v * PV;
-                const int hx = v / (HY * HZ), r = v - hx * (HY * HZ), hy = r / HZ, hz = r - hy * HZ;
-                const int gx = wrap1(bx * BX + hx - 1, n0), gy = wrap1(by * BY + hy - 1, n1);
-                const int gz = wrap1(bz * BZ + hz - 1, n2);
-                const long long gv = ((long long)gx * n1 + gy) * n2 + gz;
-                pre[j] = *(const uint2*)(a.x + gv * CIN + p * 4);
-            }
-        }
-    };
-
     const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) & 3;
     const int m = lane & 15, kq = lane >> 4;
     unsigned char* hx_ = sx[half];
-    if (2 * (int)blockIdx.x + half < nbricks) fetch(2 * blockIdx.x + half);
-    for (int pr = blockIdx.x; 2 * pr < nbricks; pr += gridDim.x) {
+
+    // 16-byte piece p of row r lies at piece p ^ swz(r): the 16 lanes that read one piece of 16
+    // consecutive rows then touch every bank once
+    auto swz = [](int r) { return CIN == 32 ? (r >> 2) & 3 : (r >> 3) & 1; };
+
+    // the next brick's halo travels in registers while the current brick computes: this thread
+    // moves piece (fz, fp) of rows RPI j + fq
+    const int fq = ht / TPR, fr = ht - fq * TPR, fz = fr / PV, fp = fr - fz * PV;
+    const bool mover = ht < 216;
+    v4u pre[NJ];
+    auto fetch = [&](int bb) {
+        const int bz = bb % nbz, by = (bb / nbz) % nby, bx = bb / (nbz * nby);
+        if (!mover) return;
+        const int gz = wrap1(bz * BZ + fz - 1, n2);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            // (rows that divide the plane evenly leave hx a constant)
+            const int row = j * RPI + fq, hx = HY % RPI == 0 ? j * RPI / HY : row / HY, hy = row - hx * HY;
+            const int gx = wrap1(bx * BX + hx - 1, n0), gy = wrap1(by * BY + hy - 1, n1);
+            pre[j] = *(const v4u*)(a.x + (((long long)gx * n1 + gy) * n2 + gz) * CIN + fp * 8);
+        }
+    };
+
+    const int npairs = (nbricks + 1) / 2, lb = xcd_rank(blockIdx.x, gridDim.x);
+    const int p_lo = (int)((long long)lb * npairs / gridDim.x), p_hi = (int)((long long)(lb + 1) * npairs / gridDim.x);
+    if (p_lo < p_hi && 2 * p_lo + half < nbricks) fetch(2 * p_lo + half);
+    {
+        constexpr int NP = 27 * COUT * PV, NW = (NP + 511) / 512;
+        v4u q[NW];
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+            const int i = threadIdx.x + j * 512;
+            if (i < NP) q[j] = *(const v4u*)(a.w + (long long)i * 8);
+        }
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+            const int i = threadIdx.x + j * 512, row = i / PV, p = i - row * PV;
+            if (i < NP) *(v4u*)(sw + row * RB + ((p ^ swz(row & 15)) * 16)) = q[j];
+        }
+    }
+
+    // lane offsets of the operands: weights row m, voxel z m + dz; slice s adds 32 bytes before the swizzle
+    auto piece = [&](int r, int s) {
+        if constexpr (K32) return r * RB + ((kq ^ swz(r)) * 16);
+        else return r * RB + (((2 * s + (kq >> 1)) ^ swz(r)) * 16) + (kq & 1) * 8;
+    };
+    int wo[NS], xo[3][NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        wo[s] = piece(m, s);
+#pragma unroll
+        for (int dz = 0; dz < 3; ++dz) xo[dz][s] = piece(m + dz, s) + w * HY * HZ * RB;
+    }
+
+    // the channels of this lane's results after the exchange below
+    const bool hi = NT == 2 && m >= 8;
+    const int c0 = (hi ? 16 : 0) + 4 * kq;
+    v4f bias = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    if (a.bias) bias = *(const v4f*)(a.bias + c0);
+
+    for (int pr = p_lo; pr < p_hi; ++pr) {
         const int bb = 2 * pr + half;
         const bool mine = bb < nbricks;
-        __syncthreads();  // the previous bricks' halo reads are done (and the weights are in)
-        if (mine) {
+        __syncthreads();  // the previous bricks' halo reads are done
+        if (mine && mover) {
 #pragma unroll
-            for (int j = 0; j < NH; ++j) {
-                const int i = ht + j * 256;
-                if (i < NP) {
-                    const int v = i / PV, p = i - v * PV;
-                    *(uint2*)(hx_ + v * SV + p * 8) = pre[j];
-                }
-            }
+            for (int j = 0; j < NJ; ++j)
+                *(v4u*)(hx_ + ((j * RPI + fq) * HZ + fz) * RB + ((fp ^ swz(fz)) * 16)) = pre[j];
         }
         __syncthreads();
-        const int nb = 2 * (pr + (int)gridDim.x) + half;
-        if (nb < nbricks) fetch(nb);
+        if (pr + 1 < p_hi && bb + 2 < nbricks) fetch(bb + 2);
         if (!mine) continue;
         const int bz = bb % nbz, by = (bb / nbz) % nby, bx = bb / (nbz * nby);
-        const int x0 = bx * BX, y0 = by * BY, z0 = bz * BZ;
+        // this lane's results of row y: NT values of 4 channels, at offset o + y n2 COUT, the
+        // second 8 voxels further
+        const long long o = ((((long long)bx * BX + w) * n1 + by * BY) * n2 + bz * BZ + (hi ? m - 8 : m)) * COUT + c0;
+        v4f res[BY][NT];
+        if (a.res)
+#pragma unroll
+            for (int y = 0; y < BY; ++y)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) res[y][t] = *(const v4f*)(a.res + o + ((long long)y * n2 + 8 * t) * COUT);
 
         v4f acc[BY][NT];
 #pragma unroll
@@ -169,99 +230,74 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) acc[y][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-        for (int dx = 0; dx < 3; ++dx)
-            for (int dy = 0; dy < 3; ++dy) {
+        // The taps of a result go in the order dx, dy, dz.  A plane's row is read once for its
+        // three dy (rows r of xf at dz; a plane's rows at dz are dead when the next plane's are
+        // read), and every tap's operands are read while the tap before it computes: left to
+        // itself the compiler reads a tap's weights one MFMA ahead and waits for each of them.
+        F xf[HY][3][NS], wf[2][NT][NS];
+        auto read_tap = [&](int tap) {
+            const int dx = tap / 9, dy = tap / 3 % 3, dz = tap % 3;
 #pragma unroll
-                for (int dz = 0; dz < 3; ++dz) {
-                    const int tap = (dx * 3 + dy) * 3 + dz;
-                    if constexpr (CIN % 32 == 0 && COUT >= 32) {
-                        // 32 input channels per MFMA (v_mfma_f32_16x16x32_bf16): lane (m, kq)
-                        // holds channels 8 kq .. 8 kq + 7 of its row / column
+            for (int t = 0; t < NT; ++t)
 #pragma unroll
-                        for (int s2 = 0; s2 < CIN / 32; ++s2) {
-                            v8bf bf[NT];
+                for (int s = 0; s < NS; ++s) wf[tap & 1][t][s] = *(const F*)(sw + wo[s] + (tap * COUT + t * 16) * RB);
 #pragma unroll
-                            for (int t = 0; t < NT; ++t)
-                                bf[t] = lds8(sw + (tap * COUT + t * 16 + m) * SV + (s2 * 32 + kq * 8) * 2);
+            for (int r = dy == 0 ? 0 : dy + BY - 1; r < dy + BY; ++r)
 #pragma unroll
-                            for (int y = 0; y < BY; ++y) {
-                                const int hv = ((w + dx) * HY + (y + dy)) * HZ + (m + dz);
-                                const v8bf af = lds8(hx_ + hv * SV + (s2 * 32 + kq * 8) * 2);
+                for (int s = 0; s < NS; ++s) xf[r][dz][s] = *(const F*)(hx_ + xo[dz][s] + (dx * HY + r) * HZ * RB);
+        };
+        read_tap(0);
 #pragma unroll
-                                for (int t = 0; t < NT; ++t)
-                                    acc[y][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bf[t], acc[y][t], 0, 0, 0);
-                            }
-                        }
-                    } else {
+        for (int tap = 0; tap < 27; ++tap) {
+            const int dy = tap / 3 % 3, dz = tap % 3;
+            if (tap < 26) read_tap(tap + 1);
 #pragma unroll
-                        for (int s2 = 0; s2 < CIN / 16; ++s2) {
-                            v4s bf[NT];
+            for (int s = 0; s < NS; ++s)
 #pragma unroll
-                            for (int t = 0; t < NT; ++t)
-                                bf[t] = *(const v4s*)(sw + (tap * COUT + t * 16 + m) * SV + (s2 * 16 + kq * 4) * 2);
+                for (int y = 0; y < BY; ++y)
 #pragma unroll
-                            for (int y = 0; y < BY; ++y) {
-                                const int hv = ((w + dx) * HY + (y + dy)) * HZ + (m + dz);
-                                const v4s af = *(const v4s*)(hx_ + hv * SV + (s2 * 16 + kq * 4) * 2);
+                    for (int t = 0; t < NT; ++t) acc[y][t] = mma(wf[tap & 1][t][s], xf[y + dy][dz][s], acc[y][t]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+        // D[row = output channel (t 16 + 4 kq + j)][col = voxel z m].  With 32 output channels,
+        // lanes m and m ^ 8 swap one result (a DPP rotation of the 16 lanes by 8): lanes below 8
+        // then hold channels 4 kq .. + 3 of voxels m and m + 8, the others channels 16 + 4 kq .. + 3
+        // of voxels m - 8 and m, and one 16-byte store instruction covers 8 whole 32-channel rows
+        // (a row's halves from two instructions reach memory as partial lines).
 #pragma unroll
-                                for (int t = 0; t < NT; ++t)
-                                    acc[y][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bf[t], acc[y][t], 0, 0, 0);
-                            }
-                        }
-                    }
+        for (int y = 0; y < BY; ++y) {
+            v4f v[NT];
+            if constexpr (NT == 2) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float give = hi ? acc[y][0][j] : acc[y][1][j];
+                    const float got =
+                        __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0x128, 0xF, 0xF, false));
+                    v[0][j] = hi ? got : acc[y][0][j];
+                    v[1][j] = hi ? acc[y][1][j] : got;
+                }
+            } else {
+                v[0] = acc[y][0];
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const long long at = o + ((long long)y * n2 + 8 * t) * COUT;
+                v[t] += bias;
+                if (a.zs) {
+                    const v4f z = *(const v4f*)(a.zs + at);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[t][j] *= dsilu(z[j]);
+                }
+                if (a.res) v[t] += res[y][t];
+                if (a.outf) *(v4f*)(a.outf + at) = v[t];
+                if (a.outb) {
+                    if (a.act)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[t][j] = silu(v[t][j]);
+                    *(v4bf*)(a.outb + at) = __builtin_convertvector(v[t], v4bf);  // v_cvt_pk_bf16_f32
                 }
             }
-
-        // D[row = z (4 kq + j)][col = output channel (t 16 + m)]
-        if constexpr (NT == 2) {
-            // lanes m and m ^ 1 swap one value (DPP quad permute 1,0,3,2): the even lane then
-            // holds channels m, m + 1 and the odd lane 15 + m, 16 + m of the same voxel, and
-            // each stores its pair at once, so a store instruction covers each voxel's whole
-            // 32-channel row (128 B in FP32, 64 B in BF16) instead of two halves
-            const bool odd = (m & 1) != 0;
-            const long long vb0 = (((long long)(x0 + w) * n1 + y0) * n2 + z0 + kq * 4) * COUT;  // channel 0
-            const float b0 = a.bias ? a.bias[m] : 0.0f, b1 = a.bias ? a.bias[16 + m] : 0.0f;
-#pragma unroll
-            for (int y = 0; y < BY; ++y)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const long long vb = vb0 + ((long long)y * n2 + j) * COUT;
-                    float v0 = acc[y][0][j] + b0, v1 = acc[y][1][j] + b1;
-                    if (a.zs) {
-                        v0 *= dsilu(a.zs[vb + m]);
-                        v1 *= dsilu(a.zs[vb + 16 + m]);
-                    }
-                    if (a.res) {
-                        v0 += a.res[vb + m];
-                        v1 += a.res[vb + 16 + m];
-                    }
-                    const float give = odd ? v0 : v1;
-                    const float got =
-                        __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0xB1, 0xF, 0xF, false));
-                    const float plo = odd ? got : v0, phi = odd ? v1 : got;
-                    const long long o = vb + (odd ? 15 + m : m);  // even: 8-byte aligned
-                    if (a.outf) *(float2*)(a.outf + o) = make_float2(plo, phi);
-                    if (a.outb)
-                        *(uint32_t*)(a.outb + o) = (uint32_t)f2bf(a.act ? silu(plo) : plo) |
-                                                   ((uint32_t)f2bf(a.act ? silu(phi) : phi) << 16);
-                }
-            continue;
-        }
-        const long long ob = (((long long)(x0 + w) * n1 + y0) * n2 + z0 + kq * 4) * COUT + m;  // (t, y, j) = 0
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const float bias = a.bias ? a.bias[t * 16 + m] : 0.0f;
-#pragma unroll
-            for (int y = 0; y < BY; ++y)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const long long o = ob + ((long long)y * n2 + j) * COUT + t * 16;
-                    float v = acc[y][t][j] + bias;
-                    if (a.zs) v *= dsilu(a.zs[o]);
-                    if (a.res) v += a.res[o];
-                    if (a.outf) a.outf[o] = v;
-                    if (a.outb) a.outb[o] = f2bf(a.act ? silu(v) : v);
-                }
         }
     }
 }
@@ -315,10 +351,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_wgrad(WgradArgs a, int nbricks) 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int dx = w / 3, dz = w % 3;
     const int i16 = lane & 15, kq = lane >> 4;
-    // contiguous brick range of this block; consecutive ranges on one XCD (blocks are dealt
-    // round-robin over the 8 XCDs)
-    const int nb = gridDim.x, per = nb / 8, rem = nb % 8, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int lb = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+    const int nb = gridDim.x, lb = xcd_rank(blockIdx.x, nb);
     const int b_lo = (int)((long long)lb * nbricks / nb), b_hi = (int)((long long)(lb + 1) * nbricks / nb);
 
     v4u px[NX], py[NY];
@@ -721,12 +754,20 @@ template <int CIN, int COUT>
 int conv(const int32_t n[3], const uint16_t* x, const uint16_t* w, const float* bias, const float* zs,
          const float* res, float* outf, uint16_t* outb, int act, hipStream_t st) {
     ConvArgs a{{n[0], n[1], n[2]}, x, w, bias, zs, res, outf, outb, act};
-    const int bricks = (n[0] / BX) * (n[1] / BY) * (n[2] / BZ);
-    // one persistent block per CU: the weights are staged in LDS once per block, and its two
-    // halves work on two bricks at a time
-    const int pairs = (bricks + 1) / 2;
-    const int blocks = pairs < cu_count() ? pairs : cu_count();
-    hipLaunchKernelGGL((k_conv<CIN, COUT>), dim3(blocks), dim3(512), 0, st, a, bricks);
+    // One persistent block per CU: the weights are staged in LDS once per block, and its two
+    // halves work on two bricks at a time.  Bricks of 4 or of 2 rows: a round of bricks costs about
+    // its rows and two rows' time for the halo and the latency, so the shorter ones pay where
+    // the taller ones leave halves idle (32^3, 128 tall bricks for 512 halves: 7.7 against 9.0 us,
+    // first conv of a block) and not in whole rounds (64^3: 23.9 against 19.2 us) or nearly so
+    // (36 x 60 x 64, 540 tall bricks: 17.8 against 16.8 us).
+    const int planes = (n[0] / BX) * (n[2] / BZ), halves = 2 * cu_count();
+    auto rounds = [&](int rows) { return (planes * (n[1] / rows) + halves - 1) / halves; };
+    auto go = [&](auto kernel, int rows) {
+        const int bricks = planes * (n[1] / rows), pairs = (bricks + 1) / 2;
+        hipLaunchKernelGGL(kernel, dim3(std::min(pairs, cu_count())), dim3(512), 0, st, a, bricks);
+    };
+    if (2 * rounds(2) < 3 * rounds(4)) go(k_conv<CIN, COUT, 2>, 2);
+    else go(k_conv<CIN, COUT, 4>, 4);
     NOPCK(hipGetLastError());
     return 0;
 }
