@@ -1255,17 +1255,26 @@ __device__ __forceinline__ float4 sum_partials(const FieldArgs& F, int i, int x,
 }
 
 // The block slices of a tile (grids of few tiles split each tile among nsl blocks) summed in
-// FP64 into the tile's first slice, one thread per partial entry: the node sums then read one
-// slice per tile instead of nsl.
+// FP64 into the tile's first slice: the node sums then read one slice per tile instead of nsl.
+// 32 entries x 8 groups of slices per block: with one thread per entry a tile's 2187 entries are
+// 9 blocks, each thread in a chain of nsl dependent reads (8^3 cells, nsl 128: 32 us
+// against 3.1 us so).
 __global__ __launch_bounds__(256) void k_slice_sum(Geo g, float* jpart) {
-    const long long per = 3LL * g.NJ;
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)g.ntiles * per) return;
-    const long long t = i / per, e = i - t * per;
-    float* base = jpart + t * g.nsl * per + e;
+    __shared__ double s_acc[8][32];
+    const int per = 3 * g.NJ, groups = (per + 31) / 32;
+    const int t = blockIdx.x / groups, c = threadIdx.x & 31, q = threadIdx.x >> 5;
+    const int e = (blockIdx.x - t * groups) * 32 + c;
+    float* base = jpart + (long long)t * g.nsl * per + e;
     double acc = 0.0;
-    for (int s = 0; s < g.nsl; ++s) acc += (double)base[s * per];
-    base[0] = (float)acc;
+    if (e < per)
+#pragma unroll 8
+        for (int s = q; s < g.nsl; s += 8) acc += (double)base[(long long)s * per];
+    s_acc[q][c] = acc;
+    __syncthreads();
+    if (q == 0 && e < per) {
+        for (int k = 1; k < 8; ++k) acc += s_acc[k][c];
+        base[0] = (float)acc;
+    }
 }
 
 // J from the tile partials, without a field update (ahead of the field operator).
@@ -1425,7 +1434,6 @@ struct ScanSp {
     int* stay;
     int* arr;
     int* tile_total;
-    int* tile_base;
 };
 struct ScanArgs {
     Geo g;
@@ -1454,9 +1462,10 @@ __global__ __launch_bounds__(NT) void k_scan_tiles(ScanArgs A) {
 // same results: the order only schedules.
 __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul) {
     const Geo& g = A.g;
-    __shared__ unsigned long long s_sum[16];
-    __shared__ int s_max[16], s_w4[4];
+    __shared__ unsigned long long s_sum[NT / 64];
+    __shared__ int s_max[NT / 64], s_w4[NT / 64];
     __shared__ int s_hist[256];
+    static_assert(NT == 256, "one thread per load class");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     auto load = [&](int t) {
         int v = 0;
@@ -1465,7 +1474,7 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul
     };
     unsigned long long sum = 0;
     int mx = 0;
-    for (int t = tid; t < g.ntiles; t += 1024) {
+    for (int t = tid; t < g.ntiles; t += NT) {
         const int v = load(t);
         sum += (unsigned long long)v;
         mx = max(mx, v);
@@ -1479,78 +1488,41 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul
         s_sum[wid] = sum;
         s_max[wid] = mx;
     }
-    if (tid < 256) s_hist[tid] = 0;
+    s_hist[tid] = 0;
     __syncthreads();
     sum = 0;
     mx = 0;
-    for (int w = 0; w < 16; ++w) {
+    for (int w = 0; w < NT / 64; ++w) {
         sum += s_sum[w];
         mx = max(mx, s_max[w]);
     }
     if ((double)mx * g.ntiles <= 1.25 * (double)sum || mx == 0) {
-        for (int b = tid; b < g.ntiles; b += 1024) order[b] = (int)(((long long)b * mul) % g.ntiles);
+        for (int b = tid; b < g.ntiles; b += NT) order[b] = (int)(((long long)b * mul) % g.ntiles);
         return;
     }
     auto cls = [&](int v) { return 255 - (int)(((long long)v * 255) / mx); };  // heaviest: class 0
-    for (int t = tid; t < g.ntiles; t += 1024) atomicAdd(&s_hist[cls(load(t))], 1);
+    for (int t = tid; t < g.ntiles; t += NT) atomicAdd(&s_hist[cls(load(t))], 1);
     __syncthreads();
-    // exclusive prefix sum of the 256 class counts, by the first four waves
-    int c = 0, incl = 0;
-    if (tid < 256) {
-        c = s_hist[tid];
-        incl = wave_incl_scan(c, lane);
-        if (lane == 63) s_w4[wid] = incl;
-    }
+    int tot;  // exclusive prefix sum of the 256 class counts
+    const int first = block_exscan(s_hist[tid], s_w4, tot);
+    s_hist[tid] = first;
     __syncthreads();
-    if (tid < 256) {
-        int off = 0;
-        for (int w = 0; w < wid; ++w) off += s_w4[w];
-        s_hist[tid] = off + incl - c;
-    }
-    __syncthreads();
-    for (int t = tid; t < g.ntiles; t += 1024) order[atomicAdd(&s_hist[cls(load(t))], 1)] = t;
-}
-
-// Tile bases from the tile totals, one block per species; block nsp (the last) orders the
-// tiles for the next push meanwhile.
-__global__ __launch_bounds__(1024) void k_scan_top(ScanArgs A, int nsp, int* order, int mul) {
-    if ((int)blockIdx.x == nsp) {
-        tile_order_block(A, nsp, order, mul);
-        return;
-    }
-    const Geo& g = A.g;
-    const ScanSp& S = A.sp[blockIdx.x];
-    __shared__ int s_part[1024];
-    const int per = (g.ntiles + 1023) / 1024;
-    const int b0 = threadIdx.x * per;
-    int v = 0;
-    for (int k = 0; k < per; ++k)
-        if (b0 + k < g.ntiles) v += S.tile_total[b0 + k];
-    s_part[threadIdx.x] = v;
-    __syncthreads();
-    // Hillis-Steele inclusive scan over 1024 partial sums
-    for (int d = 1; d < 1024; d <<= 1) {
-        const int y = threadIdx.x >= d ? s_part[threadIdx.x - d] : 0;
-        __syncthreads();
-        s_part[threadIdx.x] += y;
-        __syncthreads();
-    }
-    int run = s_part[threadIdx.x] - v;
-    for (int k = 0; k < per; ++k)
-        if (b0 + k < g.ntiles) {
-            S.tile_base[b0 + k] = run;
-            run += S.tile_total[b0 + k];
-        }
-    if (threadIdx.x == 1023) S.tile_base[g.ntiles] = s_part[1023];
+    for (int t = tid; t < g.ntiles; t += NT) order[atomicAdd(&s_hist[cls(load(t))], 1)] = t;
 }
 
 // New starts = tile base + in-tile exclusive prefix of the counts, written over the old
 // segments; the host then swaps `seg` and `start` (the previous starts become the segments of
 // the array just written, without a copy) and `stay` and `stay_acc` (the stayer counts become
 // `stay`; the old `stay`, cleared here, the next accumulator).  The cell counters and arrival
-// counters are cleared for the next pass.
-__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A) {
+// counters are cleared for the next pass.  Every block adds up the totals of the tiles before its
+// own (16 KB at most from L2 at 128^3): a launch for the bases alone costs more than these reads.
+// A further block orders the tiles for the next push meanwhile.
+__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order, int mul) {
     const Geo& g = A.g;
+    if ((int)blockIdx.x == g.ntiles) {
+        if (blockIdx.y == 0) tile_order_block(A, nsp, order, mul);
+        return;
+    }
     const ScanSp& S = A.sp[blockIdx.y];
     __shared__ int s_w[NT / 64];
     const int t = blockIdx.x;
@@ -1559,8 +1531,12 @@ __global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A) {
     int v0 = 0, v1 = 0;
     if (c0 < g.TC) v0 = S.cnt_acc[id0];
     if (c1 < g.TC) v1 = S.cnt_acc[id1];
-    int tot;
-    const int ex = block_exscan(v0 + v1, s_w, tot) + S.tile_base[t];
+    int before = 0;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < t; k += NT) before += S.tile_total[k];
+    int tot, base;
+    block_exscan(before, s_w, base);
+    const int ex = block_exscan(v0 + v1, s_w, tot) + base;
     if (c0 < g.TC) {
         S.seg[id0] = ex;
         S.stay[id0] = 0;
@@ -1573,9 +1549,42 @@ __global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A) {
         S.cnt_acc[id1] = 0;
         S.arr[id1] = 0;
     }
-    if (t == g.ntiles - 1 && threadIdx.x == 0) S.seg[g.ncell] = S.tile_base[g.ntiles];
+    if (t == g.ntiles - 1 && threadIdx.x == 0) S.seg[g.ncell] = base + tot;
 }
 
+// The same for a grid of few cells, in one launch of one block per species: each wave takes a
+// contiguous share of the cells, adds it up, and scans it 64 cells at a time from the shares before.
+// No tile order: with few tiles every block of the next push is resident at once.
+constexpr int SCAN_SMALL = 12288;  // cells up to which this is faster (see launch_scan)
+
+__global__ __launch_bounds__(1024) void k_scan_small(ScanArgs A) {
+    const int ncell = A.g.ncell;
+    const ScanSp& S = A.sp[blockIdx.x];
+    __shared__ int s_w[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int share = ((ncell + 15) / 16 + 63) & ~63, lo = min(w * share, ncell), hi = min(lo + share, ncell);
+    int v = 0;
+#pragma unroll 8
+    for (int i = lo + lane; i < hi; i += 64) v += S.cnt_acc[i];
+    v = wave_incl_scan(v, lane);
+    if (lane == 63) s_w[w] = v;
+    __syncthreads();
+    int run = 0;
+    for (int k = 0; k < w; ++k) run += s_w[k];
+#pragma unroll 4
+    for (int i0 = lo; i0 < hi; i0 += 64) {
+        const int i = i0 + lane, c = i < hi ? S.cnt_acc[i] : 0;
+        const int incl = wave_incl_scan(c, lane);
+        if (i < hi) {
+            S.seg[i] = run + incl - c;
+            S.stay[i] = 0;
+            S.cnt_acc[i] = 0;
+            S.arr[i] = 0;
+        }
+        run += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (w == 15 && lane == 0) S.seg[ncell] = run;
+}
 
 // After a REBIN pass the array is sorted by current cell: segments = starts, all stay.
 __global__ __launch_bounds__(256) void k_canon_fix(ScanArgs A) {
@@ -2023,7 +2032,6 @@ struct Species {
     int* stay_acc = nullptr;
     int* arr = nullptr;
     int* tile_total = nullptr;
-    int* tile_base = nullptr;
     int* work = nullptr;  // cells whose arrivals k_canon_large orders (IPIC_FLAG_REPRODUCIBLE)
 };
 
@@ -2206,7 +2214,7 @@ ScanArgs scan_args(ipic_ctx* ctx) {
     A.g = ctx->g;
     for (int s = 0; s < ctx->d.nspecies; ++s) {
         Species& S = ctx->sp[s];
-        A.sp[s] = ScanSp{S.cnt_acc, S.stay_acc, S.seg, S.start, S.stay, S.arr, S.tile_total, S.tile_base};
+        A.sp[s] = ScanSp{S.cnt_acc, S.stay_acc, S.seg, S.start, S.stay, S.arr, S.tile_total};
     }
     return A;
 }
@@ -2271,15 +2279,23 @@ int launch_particles(ipic_ctx* ctx, int mode) {
 int launch_scan(ipic_ctx* ctx) {
     ScanArgs A = scan_args(ctx);
     const int ns = ctx->d.nspecies;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(ctx->g.ntiles, ns), dim3(NT), 0, ctx->stream, A);
-    hipLaunchKernelGGL(k_scan_top, dim3(ns + 1), dim3(1024), 0, ctx->stream, A, ns, ctx->tile_order, ctx->order_mul);
-    hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles, ns), dim3(NT), 0, ctx->stream, A);
+    // One launch where a block per species does it in less than two launches take and the gap between
+    // them (one species, 16^3 cells: 4.1 us, 20^3: 5.5, 24^3: 8.0, 32^3: 12.9; the two launches: 8.3
+    // us and a gap at 24^3, 8.9 at 32^3).
+    const bool small = ctx->g.ncell <= SCAN_SMALL;
+    if (small) {
+        hipLaunchKernelGGL(k_scan_small, dim3(ns), dim3(1024), 0, ctx->stream, A);
+    } else {
+        hipLaunchKernelGGL(k_scan_tiles, dim3(ctx->g.ntiles, ns), dim3(NT), 0, ctx->stream, A);
+        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order,
+                           ctx->order_mul);
+    }
     HIPCK(ctx, hipGetLastError());
     for (int s = 0; s < ns; ++s) {  // the roles k_scan_cells gave the arrays
         std::swap(ctx->sp[s].seg, ctx->sp[s].start);
         std::swap(ctx->sp[s].stay, ctx->sp[s].stay_acc);
     }
-    ctx->order_valid = true;
+    ctx->order_valid = !small;
     return 0;
 }
 
@@ -2310,8 +2326,8 @@ int launch_jsum(ipic_ctx* ctx);
 int slice_sum(ipic_ctx* ctx, FieldArgs& F) {
     const Geo& g = ctx->g;
     if (g.nsl > 1) {
-        const long long n = (long long)g.ntiles * 3 * g.NJ;
-        hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, g, ctx->jpart);
+        hipLaunchKernelGGL(k_slice_sum, dim3(g.ntiles * ((3 * g.NJ + 31) / 32)), dim3(256), 0, ctx->stream, g,
+                           ctx->jpart);
         HIPCK(ctx, hipGetLastError());
     }
     F.nsl_read = 1;
@@ -2499,7 +2515,9 @@ int field_phase(ipic_ctx* ctx, bool use_op, ipic_step_stats* st) {
     } else {
         if (int rc = launch_leapfrog(ctx)) return rc;
     }
-    if (int rc = launch_c2n(ctx)) return rc;
+    // a static field keeps the node B that the upload formed
+    if (ctx->d.field_substeps > 0)
+        if (int rc = launch_c2n(ctx)) return rc;
     if (timing) {
         HIPCK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
         if (st) st->ms_field += ev_ms(ctx, 2, 3);
@@ -2844,7 +2862,6 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             rc = rc ? rc : dalloc(ctx, &S.stay_acc, nc);
             rc = rc ? rc : dalloc(ctx, &S.arr, nc);
             rc = rc ? rc : dalloc(ctx, &S.tile_total, (size_t)g.ntiles);
-            rc = rc ? rc : dalloc(ctx, &S.tile_base, (size_t)g.ntiles + 1);
             if (d.flags & IPIC_FLAG_REPRODUCIBLE) rc = rc ? rc : dalloc(ctx, &S.work, nc + 1);
         }
         if (!rc) {
