@@ -55,7 +55,7 @@ constexpr int NW = NTP / WS;     // waves per block of the particle kernel
 constexpr int KRUN = IPIC_KRUN;
 constexpr int WCH = WS * KRUN;   // max particles per wave chunk
 constexpr int K0CAP = 32;        // leaver buffer entries per wave chunk
-constexpr int QCAP = WCH + WS;   // arrival queue entries per wave (fewer than WS carried over + one chunk)
+constexpr int QCAP = WS;         // arrival queue entries per wave
 constexpr int TCMAX = 512;       // max cells per tile
 constexpr int NJMAX = 11 * 11 * 11;  // max J nodes per tile ((T+1+2h)^3, T <= 8, h <= 1)
 constexpr int JPMAX = 4;         // max (tile, local) pairs per axis coordinate
@@ -141,12 +141,17 @@ __device__ __forceinline__ int dcell(float o) {
     return 0;
 }
 
+__device__ __forceinline__ int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+
+// i mod n in [0, n) for |i| < 2^23 and n <= 2^21.  Moves of a grid length or more take the rounded
+// quotient, at most one off (its error is below 2^-22 of a quotient below 2^23 / n), and one
+// correction either way.  (An integer division here, inlined at every use, made up half of the
+// particle kernel's 178 KB of code, more than twice the instruction cache.)
 __device__ __forceinline__ int wrapc(int i, int n) {
     if ((unsigned)i < (unsigned)n) return i;
-    if (i < 0 && i >= -n) return i + n;
-    if (i >= n && i < 2 * n) return i - n;
-    const int r = i % n;
-    return r < 0 ? r + n : r;
+    const int q = (int)floorf((float)i * __builtin_amdgcn_rcpf((float)n));
+    const int r = i - q * n;
+    return r < 0 ? r + n : (r >= n ? r - n : r);
 }
 
 // floor(a / b) for 0 <= a < 2^21 and b >= 1 through a reciprocal inv_b within one ulp of 1/b:
@@ -293,35 +298,41 @@ __device__ __forceinline__ void deposit_direct(const PushArgs& A, const TG& G, l
     const Geo& g = A.g;
     // every corner value is at most max |j| (the weights lie in [0, 1])
     if (!(fmaxf(fabsf(jx), fmaxf(fabsf(jy), fabsf(jz))) <= g.fix_lim)) atomicOr(A.err, ERR_JSAT);
+    const int lx = elx + JH, ly = ely + JH, lz = elz + JH;
+    if ((unsigned)lx < (unsigned)(G.nj0 - 1) && (unsigned)ly < (unsigned)(G.nj1 - 1) &&
+        (unsigned)lz < (unsigned)(G.nj2 - 1)) {  // all corners in the tile
+        const int l0 = (lx * G.nj1 + ly) * G.nj2 + lz;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int q = 0; q < 8; ++q) {
+            const int l = l0 + ((q >> 2) * G.nj1 + ((q >> 1) & 1)) * G.nj2 + (q & 1);
+            fix_add(&sJ[l], jx * wt[q], g.fix_scale);
+            fix_add(&sJ[G.NJ + l], jy * wt[q], g.fix_scale);
+            fix_add(&sJ[2 * G.NJ + l], jz * wt[q], g.fix_scale);
+        }
+        return;
+    }
+    const int wx = wrapc(x0 + elx, g.n[0]), wy = wrapc(y0 + ely, g.n[1]), wz = wrapc(z0 + elz, g.n[2]);
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const float ww = wt[(i * 2 + j) * 2 + k];
-                const int nx = elx + JH + i, ny = ely + JH + j, nz = elz + JH + k;
-                if (nx >= 0 && nx < G.nj0 && ny >= 0 && ny < G.nj1 && nz >= 0 && nz < G.nj2) {
-                    const int l = (nx * G.nj1 + ny) * G.nj2 + nz;
-                    fix_add(&sJ[l], jx * ww, g.fix_scale);
-                    fix_add(&sJ[G.NJ + l], jy * ww, g.fix_scale);
-                    fix_add(&sJ[2 * G.NJ + l], jz * ww, g.fix_scale);
-                } else {
-                    // beyond the tile: the global accumulator, in the same fixed point, so J does
-                    // not depend on the order of these adds either
-                    const int gid = nid_of(g, wrapc(x0 + elx + i, g.n[0]), wrapc(y0 + ely + j, g.n[1]),
-                                           wrapc(z0 + elz + k, g.n[2]));
-                    long long* o = A.jover + 3 * (long long)gid;
-                    // every writer stores the same value: a relaxed atomic byte store
-                    __hip_atomic_store(&A.jmark[gid], (unsigned char)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_fetch_add(o + 0, fix_of(jx * ww, g.fix_scale), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_fetch_add(o + 1, fix_of(jy * ww, g.fix_scale), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_fetch_add(o + 2, fix_of(jz * ww, g.fix_scale), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
+    for (int q = 0; q < 8; ++q) {
+        const int i = q >> 2, j = (q >> 1) & 1, k = q & 1;
+        const int nx = lx + i, ny = ly + j, nz = lz + k;
+        if (nx >= 0 && nx < G.nj0 && ny >= 0 && ny < G.nj1 && nz >= 0 && nz < G.nj2) {
+            const int l = (nx * G.nj1 + ny) * G.nj2 + nz;
+            fix_add(&sJ[l], jx * wt[q], g.fix_scale);
+            fix_add(&sJ[G.NJ + l], jy * wt[q], g.fix_scale);
+            fix_add(&sJ[2 * G.NJ + l], jz * wt[q], g.fix_scale);
+        } else {
+            // beyond the tile: the global accumulator, in the same fixed point, so J does
+            // not depend on the order of these adds either
+            const int gid = nid_of(g, wrap1(wx + i, g.n[0]), wrap1(wy + j, g.n[1]), wrap1(wz + k, g.n[2]));
+            long long* o = A.jover + 3 * (long long)gid;
+            // every writer stores the same value: a relaxed atomic byte store
+            __hip_atomic_store(&A.jmark[gid], (unsigned char)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 0, fix_of(jx * wt[q], g.fix_scale), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 1, fix_of(jy * wt[q], g.fix_scale), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 2, fix_of(jz * wt[q], g.fix_scale), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 template <class TG>
@@ -347,7 +358,7 @@ __device__ __forceinline__ void count_add(const Geo& g, const TG& G, int* s_arr,
 // per-run moments in registers and the updated particle goes directly to its slot of the output
 // array.  The corner nodes and the moments are never live together (168 VGPRs: 3 waves per
 // SIMD).  Every other particle (it sits in another cell, or leaves the
-// cell) is appended to a wave queue by ballot compaction and handled afterwards with all lanes
+// cell) is copied to a wave queue by ballot compaction and handled afterwards with all lanes
 // busy.  The tile's J accumulator (64-bit fixed point) and per-cell counters live in LDS.
 // ---------------------------------------------------------------------------------------------
 
@@ -358,14 +369,6 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 
-__device__ __forceinline__ int wave_max(int x) {
-#pragma unroll
-    for (int d = WS / 2; d > 0; d >>= 1) x = max(x, __shfl_xor(x, d, WS));
-    return x;
-}
-
-__device__ __forceinline__ int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
-
 // xyz of a float4 node value (a 12-byte load: the fourth component is padding)
 __device__ __forceinline__ float3 ld3(const float4* p) {
     struct F3 { float x, y, z; };
@@ -375,29 +378,6 @@ __device__ __forceinline__ float3 ld3(const float4* p) {
 
 __device__ __forceinline__ int ballot_rank(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
-// Trilinear interpolation written as the polynomial it expands to:
-// f(x,y,z) = c0 + c1 x + c2 y + c3 z + c4 xy + c5 xz + c6 yz + c7 xyz for corner values
-// f[(i*2+j)*2+k] with the weights (i?x:1-x)(j?y:1-y)(k?z:1-z) of cell.h:876-880.
-// `add` is added to every corner value and the result is multiplied by `scale`.
-__device__ __forceinline__ void tri_coef(const float f[8], float add, float scale, float c[8]) {
-    c[0] = (f[0] + add) * scale;
-    c[1] = (f[4] - f[0]) * scale;
-    c[2] = (f[2] - f[0]) * scale;
-    c[3] = (f[1] - f[0]) * scale;
-    c[4] = ((f[6] - f[4]) - (f[2] - f[0])) * scale;
-    c[5] = ((f[5] - f[4]) - (f[1] - f[0])) * scale;
-    c[6] = ((f[3] - f[2]) - (f[1] - f[0])) * scale;
-    c[7] = (((f[7] - f[6]) - (f[5] - f[4])) - ((f[3] - f[2]) - (f[1] - f[0]))) * scale;
-}
-
-__device__ __forceinline__ float tri_eval(const float c[8], float x, float y, float z) {
-    const float a = fmaf(c[1], x, c[0]);
-    const float b = fmaf(c[4], x, c[2]);
-    const float d = fmaf(c[5], x, c[3]);
-    const float e = fmaf(c[7], x, c[6]);
-    return fmaf(z, fmaf(e, y, d), fmaf(b, y, a));
 }
 
 // Moments M = sum j * {1, x, y, z, xy, xz, yz, xyz} to the 8 corner sums
@@ -601,7 +581,7 @@ struct PLayout {
     int off_f4, off_f2, off_seg, off_cnt, off_stay, off_wlo, off_wave, wave_bytes, total;
 };
 
-__host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF) {
+__host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF, bool track) {
     PLayout L;
     int o = 3 * NJ * 8;             // J, int64
     L.off_f4 = o; o += NF * 16;     // node field (Ex,Ey,Ez,Bx)
@@ -612,10 +592,10 @@ __host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF) {
     L.off_wlo = o; o += (NW + 1) * 4;
     o = (o + 15) & ~15;
     L.off_wave = o;
-    // per wave: run table (WS+1 ints), run heads (WS ints), arrival queue (QCAP ints), leaver
-    // buffer (K0CAP x 8 floats)
-    L.wave_bytes = ((WS + 1) * 4 + WS * 4 + QCAP * 4 + 15) & ~15;
-    L.wave_bytes += K0CAP * 8 * 4;
+    // per wave: arrival queue (QCAP records: offsets, velocity, cell and, when carried, id),
+    // leaver buffer (K0CAP records of 7 words; the run heads, WS ints, lie in its upper half), run
+    // table (WS+1 ints)
+    L.wave_bytes = (QCAP * (track ? 8 : 7) * 4 + K0CAP * 7 * 4 + (WS + 1) * 4 + 15) & ~15;
     o += NW * L.wave_bytes;
     L.total = o;
     return L;
@@ -645,7 +625,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     constexpr bool DIPOLE = (OPT & OPT_DIPOLE) != 0;  // analytic dipole B, E = 0: no field staging
     extern __shared__ __align__(16) unsigned char smem[];
     const PLayout L =
-        particle_layout(G.NJ, G.TC, (MODE == MODE_PUSH && !DIPOLE) ? (G.T0 + 1) * (G.T1 + 1) * (G.T2 + 1) : 0);
+        particle_layout(G.NJ, G.TC, (MODE == MODE_PUSH && !DIPOLE) ? (G.T0 + 1) * (G.T1 + 1) * (G.T2 + 1) : 0, TRACK);
     long long* sJ = (long long*)smem;
     float4* sF4 = (float4*)(smem + L.off_f4);
     float2* sF2 = (float2*)(smem + L.off_f2);
@@ -656,10 +636,12 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
 
     const int tid = threadIdx.x, lane = tid & (WS - 1), wid = tid / WS;
     unsigned char* wbase = smem + L.off_wave + wid * L.wave_bytes;
-    int* R = (int*)wbase;                                            // WS+1 ints
-    int* H = (int*)(wbase + (WS + 1) * 4);                           // WS ints
-    int* Q = (int*)(wbase + (2 * WS + 1) * 4);                       // arrival queue
-    float* K0 = (float*)(wbase + (((2 * WS + 1) * 4 + QCAP * 4 + 15) & ~15));  // leaver buffer
+    constexpr int QW = TRACK ? 8 : 7;
+    float* Q = (float*)wbase;               // arrival queue: offsets, velocity, tile cell (, id)
+    float* K0 = Q + QCAP * QW;              // leaver buffer: offsets, velocity, tile cell
+    int* R = (int*)(K0 + K0CAP * 7);        // WS+1 ints
+    int* H = (int*)(K0 + K0CAP / 2 * 7);    // WS ints; fewer than K0CAP / 2 leavers wait at a chunk's start
+    static_assert(K0CAP / 2 * 7 >= WS, "the run heads fit the leaver buffer's upper half");
 
     const int t = A.tile_order ? A.tile_order[blockIdx.x] : xcd_tile(blockIdx.x, g.ntiles);
     const int sl = blockIdx.y;  // this block's slice of the tile's cells
@@ -721,20 +703,11 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         int carry = 0;  // stayers already placed for cell c_cur (when it continues)
         const float qom = S.qom, qs = S.qs, subk = S.subk;
 
-        // A particle sitting in another cell b (an arrival of the lagged sort, input index inq):
-        // full processing by one lane.  Its input cell is the last tile cell whose segment
-        // starts at or below inq.
-        auto arrive = [&](int inq) {
-            int kc = 0, khi = G.TC - 1;
-            while (kc < khi) {
-                const int mid = (kc + khi + 1) >> 1;
-                if (s_seg[mid] <= inq) kc = mid; else khi = mid - 1;
-            }
+        // A particle of tile cell kc at offsets (ox,oy,oz) sitting in another cell b (an arrival of
+        // the lagged sort): full processing by one lane.
+        auto arrive = [&](float ox, float oy, float oz, float vx, float vy, float vz, int kc, uint32_t id) {
             int qlx, qly, qlz;
             G.split(kc, qlx, qly, qlz);
-            const unsigned vq = (unsigned)inq * 4u;
-            const float ox = ldp(rin, vq, 0), oy = ldp(rin, vq, cs), oz = ldp(rin, vq, 2 * cs);
-            float vx = ldp(rin, vq, 3 * cs), vy = ldp(rin, vq, 4 * cs), vz = ldp(rin, vq, 5 * cs);
             const int dbx = dcell(ox), dby = dcell(oy), dbz = dcell(oz);
             float px = ox - (float)dbx, py = oy - (float)dby, pz = oz - (float)dbz;
             const int blx = qlx + dbx, bly = qly + dby, blz = qlz + dbz;  // tile-local cell b
@@ -774,7 +747,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     ok = false;
                 } else {
                     store_particle(rout, cs, oidx, sunk ? NaNf : px, py, pz, vx, vy, vz);
-                    if (TRACK) S.id_out[oidx] = S.id_in[inq];
+                    if (TRACK) S.id_out[oidx] = id;
                 }
             }
             if (MODE == MODE_PUSH && sunk) {
@@ -795,7 +768,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         auto drain_leavers = [&]() {
             const int kq_n = min(kn, K0CAP);
             for (int qi = lane; qi < kq_n; qi += WS) {
-                const float* e = K0 + qi * 8;
+                const float* e = K0 + qi * 7;
                 const float px = e[0], py = e[1], pz = e[2], vx = e[3], vy = e[4], vz = e[5];
                 const int kc = __float_as_int(e[6]);  // the tile cell it left
                 int qlx, qly, qlz;
@@ -809,19 +782,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             wave_sync();
             kn = 0;
         };
-        // processes the queue's first lim entries, one per lane, and moves the rest to the front
         int qn = 0;
-        auto drain = [&](int lim) {
-            for (int qi = lane; qi < lim; qi += WS) arrive(Q[qi]);
-            if (lim > 0) {
-                const int rest = qn - lim;
-                const int v = lane < rest ? Q[lim + lane] : 0;
-                wave_sync();
-                if (lane < rest) Q[lane] = v;
-                wave_sync();
-                qn = rest;
-            }
-        };
 
         while (c_cur < chi) {
             // runs of the next 64 cells (lane l looks at cell c_cur + l)
@@ -873,26 +834,34 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             float rx[KRUN], ry[KRUN], rz[KRUN], rvx[KRUN], rvy[KRUN], rvz[KRUN];
             uint32_t rid[TRACK ? KRUN : 1];
             const unsigned vrun = (unsigned)pst * 4u;
-            // (dword loads: wider loads need aligned register tuples that push the kernel past its
-            // register budget)
+            {
+                // Four particles of an array in one 16-byte load and the fifth in one more: 12 load
+                // instructions a run instead of 30 (128^3 x 32: 1.157 -> 1.118 ms).  Slots past the
+                // run's end read its successors (0 past the buffer's end: the range check is per
+                // word) and are cleared; a lane without a slot points past the buffer.
+                static_assert(KRUN == 5, "a run is four particles and one more");
+                typedef unsigned u4 __attribute__((ext_vector_type(4)));
+                const unsigned v4o = len > 0 ? vrun : 0xfffffff0u, v1o = len > 4 ? vrun + 16u : 0xfffffff0u;
+                auto load = [&](float (&r)[KRUN], unsigned off) {
+                    const u4 q = __builtin_amdgcn_raw_buffer_load_b128(rin, v4o, off, 0);
 #pragma unroll
-            for (int jj = 0; jj < KRUN; ++jj) {
-                if (jj < len) {
-                    const unsigned vo = vrun + 4u * jj;
-                    rx[jj] = ldp(rin, vo, 0);
-                    ry[jj] = ldp(rin, vo, cs);
-                    rz[jj] = ldp(rin, vo, 2 * cs);
-                    rvx[jj] = ldp(rin, vo, 3 * cs);
-                    rvy[jj] = ldp(rin, vo, 4 * cs);
-                    rvz[jj] = ldp(rin, vo, 5 * cs);
-                    if (TRACK) rid[jj] = S.id_in[pst + jj];
-                } else {
-                    rx[jj] = ry[jj] = rz[jj] = NaNf;
-                    rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
-                    if (TRACK) rid[jj] = 0;
-                }
+                    for (int jj = 0; jj < 4; ++jj) r[jj] = __uint_as_float(q[jj]);
+                    r[4] = ldp(rin, v1o, off);
+                };
+                load(rx, 0);
+                load(ry, cs);
+                load(rz, 2 * cs);
+                load(rvx, 3 * cs);
+                load(rvy, 4 * cs);
+                load(rvz, 5 * cs);
+#pragma unroll
+                for (int jj = 0; jj < KRUN; ++jj)
+                    if (jj >= len) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
+                if (TRACK)
+#pragma unroll
+                    for (int jj = 0; jj < KRUN; ++jj) rid[jj] = jj < len ? S.id_in[pst + jj] : 0u;
             }
-            const int c = c_cur + k;
+            const int c = c_run;
             int lx, ly, lz;
             G.split(c, lx, ly, lz);
             const int ax = x0 + lx, ay = y0 + ly, az = z0 + lz;
@@ -904,13 +873,13 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
 #pragma unroll
             for (int jj = 0; jj < KRUN; ++jj)
                 if (in_cell(rx[jj], ry[jj], rz[jj])) hm |= 1u << jj;
+            hm &= (1u << len) - 1u;  // empty slots hold zeros
             const int my_stay = (MODE != MODE_DEPOSIT) ? __popc(hm) : 0;
             const int sincl = wave_incl_scan(my_stay, lane);
             const int sex = sincl - my_stay;
             const int sfirst = __shfl(sex, R[k], WS);
             const int base = (k == 0 ? carry : 0) + sex - sfirst;
 
-            int run_in = 0, rank = 0;
             // slots of the run cell's stayers lie in [0, a_lim): below its end and the capacity
             const int a_lim = min(a_end, (int)S.cap);  // S.cap < 2^31 (one buffer resource < 4 GiB)
 
@@ -918,6 +887,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             // reflection, sink); a removed particle gets a NaN x offset.  The run cell's 8 corner
             // nodes are read from LDS once per run and held in registers for this pass only, so
             // they never share the register file with the deposit moments of pass B2.
+            unsigned im = hm, sm = 0;  // home particles that end the step in the run's cell; removed ones
             if (MODE == MODE_PUSH) {
                 float4 rn4[8];
                 float2 rn2[8];
@@ -947,7 +917,11 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                         }
                         boris_move(g, qom, subk, Ex, Ey, Ez, Bx, By, Bz, vx, vy, vz, px, py, pz);
                         if (REFLECT) reflect_faces(g, ax, ay, az, px, py, pz, vx, vy, vz);
-                        bool sunk = !finite3(px, py, pz);
+                        bool sunk = false;
+                        if (!in_cell(px, py, pz)) {
+                            im &= ~(1u << jj);
+                            sunk = !finite3(px, py, pz);
+                        }
                         if (SINK && !sunk) {
                             const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
                             const float sx_ = g.origin[0] + ((float)wrapc(ax + dex, g.n[0]) + px - (float)dex) * g.w[0] - g.sink_c[0];
@@ -955,7 +929,12 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                             const float sz_ = g.origin[2] + ((float)wrapc(az + dez, g.n[2]) + pz - (float)dez) * g.w[2] - g.sink_c[2];
                             sunk = (sx_ * sx_ + sy_ * sy_ + sz_ * sz_) <= g.sink_r2;
                         }
-                        rx[jj] = sunk ? NaNf : px;
+                        if (sunk) {
+                            sm |= 1u << jj;
+                            im &= ~(1u << jj);
+                            px = NaNf;
+                        }
+                        rx[jj] = px;
                         ry[jj] = py;
                         rz[jj] = pz;
                         rvx[jj] = vx;
@@ -976,10 +955,52 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
 #pragma unroll
             for (int jj = 0; jj < KRUN; ++jj)
                 if (!((hm >> jj) & 1u) && jj < len && alive(rx[jj], ry[jj], rz[jj])) amask |= 1u << jj;
+            const bool dead = (((1u << len) - 1u) & ~hm & ~amask) != 0u || sm != 0u;
+            // Arrivals, one of every lane that has one left, wait in the queue with all their data:
+            // read again by input index when a wave of them is there, they miss L2 and cost 0.35 of
+            // the 3.9 GB of a push at 128^3 x 32 (1.118 -> 1.083 ms).  A round that does not fit is
+            // handled at once, its idle lanes taking entries from the queue.
+            for (unsigned m = amask;;) {
+                const unsigned long long bq = __ballot(m != 0);
+                if (bq == 0) break;
+                const int jl = m ? __builtin_ctz(m) : 0, nq = __popcll(bq), rank = ballot_rank(bq);
+                float e0 = rx[0], e1 = ry[0], e2 = rz[0], e3 = rvx[0], e4 = rvy[0], e5 = rvz[0];
+                uint32_t e7 = TRACK ? rid[0] : 0u;
+#pragma unroll
+                for (int jj = 1; jj < KRUN; ++jj) {
+                    const bool at = jj == jl;
+                    e0 = at ? rx[jj] : e0; e1 = at ? ry[jj] : e1; e2 = at ? rz[jj] : e2;
+                    e3 = at ? rvx[jj] : e3; e4 = at ? rvy[jj] : e4; e5 = at ? rvz[jj] : e5;
+                    if (TRACK) e7 = at ? rid[jj] : e7;
+                }
+                bool have = m != 0;
+                if (qn + nq <= QCAP) {
+                    if (have) {
+                        float* e = Q + (qn + rank) * QW;
+                        e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
+                        e[6] = __int_as_float(c);
+                        if (TRACK) e[7] = __uint_as_float(e7);
+                    }
+                    qn += nq;
+                } else {
+                    const int from = qn - 1 - (lane - rank);  // idle lanes take the queue's last entries
+                    int kc = c;
+                    if (!have && from >= 0) {
+                        const float* e = Q + from * QW;
+                        e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
+                        kc = __float_as_int(e[6]);
+                        if (TRACK) e7 = __float_as_uint(e[7]);
+                        have = true;
+                    }
+                    if (have) arrive(e0, e1, e2, e3, e4, e5, kc, e7);
+                    qn = max(0, qn - (WS - nq));
+                }
+                wave_sync();
+                m &= m - 1;
+            }
             // A run with a single slot that is not home (an arrival, or a particle removed in the
             // previous step) closes the gap: the home particles move down one register, and the
-            // run is stored like a run of home particles only.  The arrival itself is reloaded by
-            // its input index when the queue is drained.  (Not in the instances that carry particle
+            // run is stored like a run of home particles only.  (Not in the instances that carry particle
             // ids, where the extra registers would spill; they store such runs particle by
             // particle.)
             if (MODE != MODE_DEPOSIT && !TRACK) {
@@ -1000,6 +1021,9 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     if (one_gap) {
                         --len;
                         hm = (1u << len) - 1u;
+                        const unsigned lo = (1u << zg) - 1u;
+                        im = (im & lo) | ((im >> 1) & ~lo);
+                        sm = (sm & lo) | ((sm >> 1) & ~lo);
                     }
                 }
             }
@@ -1032,32 +1056,37 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                             if (jj < len) S.id_out[o0 + jj] = rid[jj];
                 }
             }
-            unsigned lmask = 0;  // this run's leavers (register positions after a closed gap)
+            if (MODE != MODE_DEPOSIT && !whole && hm) {
+                int rank = 0;
 #pragma unroll
-            for (int jj = 0; jj < KRUN; ++jj) {
-                const float px = rx[jj], py = ry[jj], pz = rz[jj];
-                const float vx = rvx[jj], vy = rvy[jj], vz = rvz[jj];
-                const bool home = (hm >> jj) & 1u;
-                if (MODE != MODE_DEPOSIT && !whole && home) {
-                    const int oidx = a_start + base + rank;
-                    ++rank;
-                    if ((unsigned)oidx >= (unsigned)a_lim) {
-                        atomicOr(A.err, ERR_SLOT);
-                    } else {
-                        store_particle(rout, cs, oidx, px, py, pz, vx, vy, vz);
-                        if (TRACK) S.id_out[oidx] = rid[jj];
+                for (int jj = 0; jj < KRUN; ++jj)
+                    if ((hm >> jj) & 1u) {
+                        const int oidx = a_start + base + rank;
+                        ++rank;
+                        if ((unsigned)oidx >= (unsigned)a_lim) {
+                            atomicOr(A.err, ERR_SLOT);
+                        } else {
+                            store_particle(rout, cs, oidx, rx[jj], ry[jj], rz[jj], rvx[jj], rvy[jj], rvz[jj]);
+                            if (TRACK) S.id_out[oidx] = rid[jj];
+                        }
                     }
+            }
+            if (MODE == MODE_PUSH && sm) atomicAdd(A.removed, (unsigned long long)__popc(sm));
+            const unsigned lmask = (MODE == MODE_PUSH) ? hm & ~im & ~sm : 0u;  // leavers: queued below
+            const int run_in = (MODE == MODE_REBIN) ? 0 : __popc(im);
+            if (MODE != MODE_REBIN) {
+                // Moments of the particles that stay: the others add zeros through their charge.
+                // Their offsets have to be finite for that, which those of removed ones are not.
+                if (__ballot(dead)) {
+#pragma unroll
+                    for (int jj = 0; jj < KRUN; ++jj)
+                        if (!((im | lmask) >> jj & 1u)) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
                 }
-                // a home particle's x offset is NaN only when pass B1 removed it
-                const bool sunk = (MODE == MODE_PUSH) && home && __builtin_isnan(px);
-                if (sunk) atomicAdd(A.removed, 1ull);
-                if (MODE != MODE_REBIN) {
-                    const bool inc = home && (MODE == MODE_DEPOSIT || in_cell(px, py, pz));
-                    if (home && !sunk && !inc) lmask |= 1u << jj;  // leaves cell a: queued below
-                    // branch-free moments: a particle that deposits elsewhere (or not at all)
-                    // adds zeros
-                    const float dx = inc ? px : 0.0f, dy = inc ? py : 0.0f, dz = inc ? pz : 0.0f;
-                    const float jx = inc ? qs * vx : 0.0f, jy = inc ? qs * vy : 0.0f, jz = inc ? qs * vz : 0.0f;
+#pragma unroll
+                for (int jj = 0; jj < KRUN; ++jj) {
+                    const float dx = rx[jj], dy = ry[jj], dz = rz[jj];
+                    const float qj = ((im >> jj) & 1u) ? qs : 0.0f;
+                    const float jx = qj * rvx[jj], jy = qj * rvy[jj], jz = qj * rvz[jj];
                     jmax = fmaxf(jmax, fmaxf(fabsf(jx), fmaxf(fabsf(jy), fabsf(jz))));
                     const float xy = dx * dy, xz = dx * dz, yz = dy * dz, xyz = xy * dz;
                     const float mono[8] = {1.0f, dx, dy, dz, xy, xz, yz, xyz};
@@ -1067,39 +1096,37 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                         mom[1][m] = fmaf(jy, mono[m], mom[1][m]);
                         mom[2][m] = fmaf(jz, mono[m], mom[2][m]);
                     }
-                    run_in += inc ? 1 : 0;
                 }
             }
-            // ballot compaction of both queues, for the chunks that have entries
-            if (__ballot((amask | lmask) != 0)) {
+            // leavers, one of every lane that has one left, wait in their buffer; without room they
+            // are handled in place
+            if (MODE == MODE_PUSH)
+                for (unsigned m = lmask;;) {
+                    const unsigned long long bk = __ballot(m != 0);
+                    if (bk == 0) break;
+                    const int jl = m ? __builtin_ctz(m) : 0;
+                    float e0 = rx[0], e1 = ry[0], e2 = rz[0], e3 = rvx[0], e4 = rvy[0], e5 = rvz[0];
 #pragma unroll
-                for (int jj = 0; jj < KRUN; ++jj) {
-                    const bool arr = (amask >> jj) & 1u, leaver = (lmask >> jj) & 1u;
-                    const unsigned long long bq = __ballot(arr);
-                    if (arr) Q[qn + ballot_rank(bq)] = pst + jj;
-                    qn += __popcll(bq);
-                    const unsigned long long bk = __ballot(leaver);
-                    if (leaver) {
-                        const float px = rx[jj], py = ry[jj], pz = rz[jj];
-                        const float vx = rvx[jj], vy = rvy[jj], vz = rvz[jj];
-                        const int slot = kn + ballot_rank(bk);
-                        if (slot < K0CAP) {
-                            float* e = K0 + slot * 8;
-                            e[0] = px; e[1] = py; e[2] = pz; e[3] = vx; e[4] = vy; e[5] = vz;
-                            e[6] = __int_as_float(c);
-                        } else {
-                            // buffer full: handle in place
-                            const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
-                            float wt[8];
-                            tri_weights(px - (float)dex, py - (float)dey, pz - (float)dez, wt);
-                            deposit_direct(A, G, sJ, x0, y0, z0, lx + dex, ly + dey, lz + dez, wt, qs * vx,
-                                           qs * vy, qs * vz);
-                            count_add(g, G, s_cnt, S.cnt_acc, x0, y0, z0, ax + dex, ay + dey, az + dez);
-                        }
+                    for (int jj = 1; jj < KRUN; ++jj) {
+                        const bool at = jj == jl;
+                        e0 = at ? rx[jj] : e0; e1 = at ? ry[jj] : e1; e2 = at ? rz[jj] : e2;
+                        e3 = at ? rvx[jj] : e3; e4 = at ? rvy[jj] : e4; e5 = at ? rvz[jj] : e5;
                     }
-                    kn += __popcll(bk);
+                    const int slot = kn + ballot_rank(bk);
+                    if (m != 0 && slot < K0CAP) {
+                        float* e = K0 + slot * 7;
+                        e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
+                        e[6] = __int_as_float(c);
+                    } else if (m != 0) {
+                        const int dex = dcell(e0), dey = dcell(e1), dez = dcell(e2);
+                        float wt[8];
+                        tri_weights(e0 - (float)dex, e1 - (float)dey, e2 - (float)dez, wt);
+                        deposit_direct(A, G, sJ, x0, y0, z0, lx + dex, ly + dey, lz + dez, wt, qs * e3, qs * e4, qs * e5);
+                        count_add(g, G, s_cnt, S.cnt_acc, x0, y0, z0, ax + dex, ay + dey, az + dez);
+                    }
+                    kn = min(kn + (int)__popcll(bk), K0CAP);
+                    m &= m - 1;
                 }
-            }
             if (MODE != MODE_REBIN && run_in > 0) {
                 if (!(jmax * (float)run_in <= g.fix_lim)) atomicOr(A.err, ERR_JSAT);
 #pragma unroll
@@ -1123,10 +1150,8 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             }
             wave_sync();
 
-            // leavers wait in their buffer until it is half full, arrivals until a whole wave of
-            // them is there
+            // leavers wait in their buffer until it is half full
             if (kn >= K0CAP / 2) drain_leavers();
-            drain(qn & ~(WS - 1));
             // advance the wave's cursor past the runs of this chunk
             const int klast = __shfl(k, nruns - 1, WS);
             if (all_runs <= WS) {
@@ -1147,7 +1172,10 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             wave_sync();
         }
         if (kn > 0) drain_leavers();  // the leavers and arrivals still queued
-        drain(qn);
+        if (lane < qn) {
+            const float* e = Q + lane * QW;
+            arrive(e[0], e[1], e[2], e[3], e[4], e[5], __float_as_int(e[6]), TRACK ? __float_as_uint(e[QW - 1]) : 0u);
+        }
         __syncthreads();
         if (MODE == MODE_PUSH) {
             for (int i = tid; i < G.TC; i += NTP) {
@@ -2256,7 +2284,7 @@ int launch_particles(ipic_ctx* ctx, int mode) {
     dim3 grid(g.ntiles, g.nsl), block(NTP);
     const bool dip = (ctx->d.flags & IPIC_FLAG_DIPOLE_MOVER) != 0;
     const size_t lds =
-        (size_t)particle_layout(g.NJ, g.TC, (mode == MODE_PUSH && !dip) ? field_nodes(g) : 0).total;
+        (size_t)particle_layout(g.NJ, g.TC, (mode == MODE_PUSH && !dip) ? field_nodes(g) : 0, ctx->track).total;
     const int opt = ((g.T[0] == 8 && g.T[1] == 8 && g.T[2] == 8) ? OPT_FIX8 : 0) | (g.sink ? OPT_SINK : 0) |
                     (g.reflect ? OPT_REFLECT : 0) | (dip ? OPT_DIPOLE : 0);
     hipStream_t st = ctx->stream;
