@@ -679,22 +679,25 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         }
         __syncthreads();
         // the block's cells [clo, chi): slice sl of g.nsl at equal particle counts; cells of
-        // wave w: [s_wlo[w], s_wlo[w+1]), the slice split again at equal particle counts
+        // wave w: [s_wlo[w], s_wlo[w+1]), the slice split again at equal particle counts.  Each
+        // cut goes to the cell boundary nearest to it: at the next one instead, a wave of a slice of
+        // four cells of about equal size often got two of them (8^3 cells, 512 per cell: 81 against
+        // 74 us).
         if (tid <= NW) {
-            auto first_ge = [&](long long target) {  // first cell c with s_seg[c] >= target
+            auto nearest = [&](long long target) {
                 int lo = 0, hi = G.TC;
-                while (lo < hi) {
+                while (lo < hi) {  // first cell c with s_seg[c] >= target
                     const int mid = (lo + hi) >> 1;
                     if (s_seg[mid] >= target) hi = mid; else lo = mid + 1;
                 }
-                return lo;
+                return lo > 0 && target - s_seg[lo - 1] < s_seg[lo] - target ? lo - 1 : lo;
             };
             const long long tot = (long long)s_seg[G.TC] - s_seg[0];
-            const int clo = (sl == 0) ? 0 : first_ge(s_seg[0] + tot * sl / g.nsl);
-            const int chi = (sl == g.nsl - 1) ? G.TC : first_ge(s_seg[0] + tot * (sl + 1) / g.nsl);
+            const int clo = (sl == 0) ? 0 : nearest(s_seg[0] + tot * sl / g.nsl);
+            const int chi = (sl == g.nsl - 1) ? G.TC : nearest(s_seg[0] + tot * (sl + 1) / g.nsl);
             const long long sub = (long long)s_seg[chi] - s_seg[clo];
             s_wlo[tid] = (tid == 0) ? clo
-                       : (tid == NW ? chi : max(clo, min(chi, first_ge(s_seg[clo] + sub * tid / NW))));
+                       : (tid == NW ? chi : max(clo, min(chi, nearest(s_seg[clo] + sub * tid / NW))));
         }
         __syncthreads();
         const int chi = s_wlo[wid + 1];
