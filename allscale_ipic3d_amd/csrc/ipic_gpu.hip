@@ -55,7 +55,8 @@ constexpr int NW = NTP / WS;     // waves per block of the particle kernel
 constexpr int KRUN = IPIC_KRUN;
 constexpr int WCH = WS * KRUN;   // max particles per wave chunk
 constexpr int K0CAP = 32;        // leaver buffer entries per wave chunk
-constexpr int QCAP = WS;         // arrival queue entries per wave
+constexpr int QCAP = 48;         // arrival queue entries per wave
+constexpr int SPG = 2;            // species a block works through between two barriers
 constexpr int TCMAX = 512;       // max cells per tile
 constexpr int NJMAX = 11 * 11 * 11;  // max J nodes per tile ((T+1+2h)^3, T <= 8, h <= 1)
 constexpr int JPMAX = 4;         // max (tile, local) pairs per axis coordinate
@@ -126,7 +127,7 @@ struct PushArgs {
     unsigned char* jmark; // jmark[i] = 1: node i holds overflow deposits
     unsigned long long* removed;
     int* err;             // set to nonzero when a consistency guard fires
-    const int* tile_order;  // block -> tile (a permutation), or null for the XCD-aware default
+    const int* tile_order;  // block -> tile (a permutation), or null for tile = block
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -166,15 +167,6 @@ __device__ __forceinline__ int cid_of(const Geo& g, int x, int y, int z) {
 
 __device__ __forceinline__ int nid_of(const Geo& g, int x, int y, int z) {
     return (x * g.n[1] + y) * g.n[2] + z;
-}
-
-// XCD-aware block -> tile map: consecutive tiles (neighbours in x-slabs) go to the same XCD
-// (blocks are dealt round-robin over the 8 XCDs), so halo nodes shared by neighbouring tiles
-// stay in one L2.
-__device__ __forceinline__ int xcd_tile(int bid, int ntiles) {
-    const int per = ntiles / 8, rem = ntiles % 8;
-    const int xcd = bid % 8, slot = bid / 8;
-    return xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
 }
 
 // Inclusive prefix sum over the wave with DPP lane moves (no LDS round trips): shifts by 1, 2,
@@ -335,15 +327,10 @@ __device__ __forceinline__ void deposit_direct(const PushArgs& A, const TG& G, l
     }
 }
 
+// one more particle in (unwrapped) cell (x,y,z)
 template <class TG>
-__device__ __forceinline__ void count_add(const Geo& g, const TG& G, int* s_arr, int* gl, int x0, int y0, int z0,
-                                          int ex, int ey, int ez) {
-    const int lx = ex - x0, ly = ey - y0, lz = ez - z0;
-    if (lx >= 0 && lx < G.T0 && ly >= 0 && ly < G.T1 && lz >= 0 && lz < G.T2) {
-        atomicAdd(&s_arr[(lx * G.T1 + ly) * G.T2 + lz], 1);
-    } else {
-        atomicAdd(&gl[G.cid(g, wrapc(ex, g.n[0]), wrapc(ey, g.n[1]), wrapc(ez, g.n[2]))], 1);
-    }
+__device__ __forceinline__ void count_in(const Geo& g, const TG& G, int* count, int x, int y, int z) {
+    atomicAdd(&count[G.cid(g, wrapc(x, g.n[0]), wrapc(y, g.n[1]), wrapc(z, g.n[2]))], 1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -578,7 +565,7 @@ __device__ __forceinline__ void gather_regs(const float4 n4[8], const float2 n2[
 
 // Dynamic LDS layout of k_particles (bytes, 16-aligned sections)
 struct PLayout {
-    int off_f4, off_f2, off_seg, off_cnt, off_stay, off_wlo, off_wave, wave_bytes, total;
+    int off_f4, off_f2, off_seg, off_cnt, off_wlo, off_wave, wave_bytes, total;
 };
 
 __host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF, bool track) {
@@ -586,10 +573,9 @@ __host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF, bool 
     int o = 3 * NJ * 8;             // J, int64
     L.off_f4 = o; o += NF * 16;     // node field (Ex,Ey,Ez,Bx)
     L.off_f2 = o; o += NF * 8;      // node field (By,Bz)
-    L.off_seg = o; o += (TC + 1) * 4;
-    L.off_cnt = o; o += TC * 4;
-    L.off_stay = o; o += TC * 4;
-    L.off_wlo = o; o += (NW + 1) * 4;
+    L.off_seg = o; o += SPG * (TC + 1) * 4;  // segment starts of SPG species
+    L.off_cnt = o; o += 2 * TC * 4;           // per cell, 16 bits for each of them: stayers, others
+    L.off_wlo = o; o += SPG * (NW + 1) * 4;
     o = (o + 15) & ~15;
     L.off_wave = o;
     // per wave: arrival queue (QCAP records: offsets, velocity, cell and, when carried, id),
@@ -629,10 +615,11 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     long long* sJ = (long long*)smem;
     float4* sF4 = (float4*)(smem + L.off_f4);
     float2* sF2 = (float2*)(smem + L.off_f2);
-    int* s_seg = (int*)(smem + L.off_seg);
-    int* s_cnt = (int*)(smem + L.off_cnt);
-    int* s_stay = (int*)(smem + L.off_stay);
-    int* s_wlo = (int*)(smem + L.off_wlo);
+    int* s_segs = (int*)(smem + L.off_seg);
+    unsigned* s_stay = (unsigned*)(smem + L.off_cnt);
+    unsigned* s_cnt = s_stay + G.TC;
+    int* s_wlos = (int*)(smem + L.off_wlo);
+    static_assert(SPG == 2, "two species share a word of stayer counts");
 
     const int tid = threadIdx.x, lane = tid & (WS - 1), wid = tid / WS;
     unsigned char* wbase = smem + L.off_wave + wid * L.wave_bytes;
@@ -643,7 +630,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     int* H = (int*)(K0 + K0CAP / 2 * 7);    // WS ints; fewer than K0CAP / 2 leavers wait at a chunk's start
     static_assert(K0CAP / 2 * 7 >= WS, "the run heads fit the leaver buffer's upper half");
 
-    const int t = A.tile_order ? A.tile_order[blockIdx.x] : xcd_tile(blockIdx.x, g.ntiles);
+    const int t = A.tile_order ? A.tile_order[blockIdx.x] : (int)blockIdx.x;
     const int sl = blockIdx.y;  // this block's slice of the tile's cells
     const int tx = t / (g.NTl[1] * g.NTl[2]), ty = (t / g.NTl[2]) % g.NTl[1], tz = t % g.NTl[2];
     const int x0 = tx * G.T0, y0 = ty * G.T1, z0 = tz * G.T2;
@@ -666,24 +653,101 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         }
     }
 
-    for (int s = 0; s < A.nsp; ++s) {
-        const SpArgs& S = A.sp[s];
-        const Rsrc rin = make_rsrc(S.in, S.cap * 24);
-        const Rsrc rout = make_rsrc(S.out, S.cap * 24);
-        const unsigned cs = (unsigned)S.cap * 4u;  // byte stride between the six arrays
-        __syncthreads();
-        for (int i = tid; i <= G.TC; i += NTP) s_seg[i] = S.seg[cbase + i];
-        for (int i = tid; i < G.TC; i += NTP) {
-            s_cnt[i] = 0;
-            s_stay[i] = 0;
+    // A particle of tile cell kc at offsets (ox,oy,oz) sitting in another cell b (an arrival of
+    // the lagged sort): full processing by one lane.  With cshift >= 0 the block's counters for
+    // species S are half words, `cshift` bits up, in LDS.
+    auto arrive = [&](const SpArgs& S, int cshift, float ox, float oy, float oz, float vx, float vy, float vz, int kc,
+                      uint32_t id) {
+        int qlx, qly, qlz;
+        G.split(kc, qlx, qly, qlz);
+        const int dbx = dcell(ox), dby = dcell(oy), dbz = dcell(oz);
+        float px = ox - (float)dbx, py = oy - (float)dby, pz = oz - (float)dbz;
+        const int blx = qlx + dbx, bly = qly + dby, blz = qlz + dbz;  // tile-local cell b
+        const int bx = x0 + blx, by = y0 + bly, bz = z0 + blz;        // unwrapped
+        const int bxw = wrapc(bx, g.n[0]), byw = wrapc(by, g.n[1]), bzw = wrapc(bz, g.n[2]);
+        // its slot first: the loads and the atomic are on their way while it is pushed
+        int bc = 0, oidx = 0, oend = 0;
+        if (MODE != MODE_DEPOSIT) {
+            bc = G.cid(g, bxw, byw, bzw);
+            oend = S.start[bc + 1];
+            oidx = S.start[bc] + S.stay[bc] + atomicAdd(&S.arr[bc], 1);
         }
+        bool sunk = false;
+        int dex = 0, dey = 0, dez = 0;
+        if (MODE == MODE_PUSH) {
+            float Ex, Ey, Ez, Bx, By, Bz;
+            if (DIPOLE) {
+                Ex = Ey = Ez = 0.0f;
+                dipole_field(g, bxw, byw, bzw, px, py, pz, Bx, By, Bz);
+            } else if ((unsigned)blx < (unsigned)G.T0 && (unsigned)bly < (unsigned)G.T1 &&
+                       (unsigned)blz < (unsigned)G.T2)
+                gather_lds(sF4, sF2, blx * fsx + bly * fsy + blz, fsx, fsy, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
+            else
+                gather_direct(A, bxw, byw, bzw, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
+            boris_move(g, S.qom, S.subk, Ex, Ey, Ez, Bx, By, Bz, vx, vy, vz, px, py, pz);
+            if (REFLECT) reflect_faces(g, bxw, byw, bzw, px, py, pz, vx, vy, vz);
+            sunk = !finite3(px, py, pz);
+            if (!sunk) {
+                dex = dcell(px); dey = dcell(py); dez = dcell(pz);
+            }
+            if (SINK && !sunk) {
+                const float rx_ = g.origin[0] + ((float)wrapc(bx + dex, g.n[0]) + px - (float)dex) * g.w[0] - g.sink_c[0];
+                const float ry_ = g.origin[1] + ((float)wrapc(by + dey, g.n[1]) + py - (float)dey) * g.w[1] - g.sink_c[1];
+                const float rz_ = g.origin[2] + ((float)wrapc(bz + dez, g.n[2]) + pz - (float)dez) * g.w[2] - g.sink_c[2];
+                sunk = (rx_ * rx_ + ry_ * ry_ + rz_ * rz_) <= g.sink_r2;
+            }
+        }
+        bool ok = true;
+        if (MODE != MODE_DEPOSIT) {
+            if (oidx < 0 || oidx >= oend || (long long)oidx >= S.cap) {
+                atomicOr(A.err, ERR_SLOT);
+                ok = false;
+            } else {
+                store_particle(make_rsrc(S.out, S.cap * 24), (unsigned)S.cap * 4u, oidx, sunk ? NaNf : px, py, pz, vx,
+                               vy, vz);
+                if (TRACK) S.id_out[oidx] = id;
+            }
+        }
+        if (MODE == MODE_PUSH && sunk) {
+            atomicAdd(A.removed, 1ull);
+        } else if (MODE != MODE_REBIN && ok) {
+            float wt[8];
+            tri_weights(px - (float)dex, py - (float)dey, pz - (float)dez, wt);
+            deposit_direct(A, G, sJ, x0, y0, z0, blx + dex, bly + dey, blz + dez, wt, S.qs * vx, S.qs * vy,
+                           S.qs * vz);
+            if (MODE == MODE_PUSH) {
+                const bool stays = (dex | dey | dez) == 0;
+                const int ex = blx + dex, ey = bly + dey, ez = blz + dez;
+                if (cshift >= 0 && (unsigned)ex < (unsigned)G.T0 && (unsigned)ey < (unsigned)G.T1 &&
+                    (unsigned)ez < (unsigned)G.T2) {
+                    atomicAdd(&(stays ? s_stay : s_cnt)[(ex * G.T1 + ey) * G.T2 + ez], 1u << cshift);
+                } else {
+                    const int ec = G.cid(g, wrapc(bx + dex, g.n[0]), wrapc(by + dey, g.n[1]), wrapc(bz + dez, g.n[2]));
+                    atomicAdd(&S.cnt_acc[ec], 1);
+                    if (stays) atomicAdd(&S.stay_acc[ec], 1);
+                }
+            }
+        }
+    };
+
+    // Up to SPG species between two barriers: their segment starts are read together, and a wave goes
+    // on with its cells of the next species when it is done.
+    for (int sg = 0; sg < A.nsp; sg += SPG) {
+        const int ns = min(SPG, A.nsp - sg);
+        if (sg > 0) __syncthreads();
+        if (MODE == MODE_PUSH)
+            for (int i = tid; i < 2 * G.TC; i += NTP) s_stay[i] = 0u;
+        for (int q = 0; q < ns; ++q)
+            for (int i = tid; i <= G.TC; i += NTP) s_segs[q * (G.TC + 1) + i] = A.sp[sg + q].seg[cbase + i];
         __syncthreads();
         // the block's cells [clo, chi): slice sl of g.nsl at equal particle counts; cells of
         // wave w: [s_wlo[w], s_wlo[w+1]), the slice split again at equal particle counts.  Each
         // cut goes to the cell boundary nearest to it: at the next one instead, a wave of a slice of
         // four cells of about equal size often got two of them (8^3 cells, 512 per cell: 81 against
         // 74 us).
-        if (tid <= NW) {
+        if (tid < ns * (NW + 1)) {
+            const int q = tid / (NW + 1), w = tid - q * (NW + 1);
+            const int* s_seg = s_segs + q * (G.TC + 1);
             auto nearest = [&](long long target) {
                 int lo = 0, hi = G.TC;
                 while (lo < hi) {  // first cell c with s_seg[c] >= target
@@ -696,494 +760,464 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
             const int clo = (sl == 0) ? 0 : nearest(s_seg[0] + tot * sl / g.nsl);
             const int chi = (sl == g.nsl - 1) ? G.TC : nearest(s_seg[0] + tot * (sl + 1) / g.nsl);
             const long long sub = (long long)s_seg[chi] - s_seg[clo];
-            s_wlo[tid] = (tid == 0) ? clo
-                       : (tid == NW ? chi : max(clo, min(chi, nearest(s_seg[clo] + sub * tid / NW))));
+            s_wlos[tid] = (w == 0) ? clo
+                        : (w == NW ? chi : max(clo, min(chi, nearest(s_seg[clo] + sub * w / NW))));
         }
         __syncthreads();
-        const int chi = s_wlo[wid + 1];
-        int c_cur = s_wlo[wid];
-        int pos_cur = s_seg[c_cur];
-        int carry = 0;  // stayers already placed for cell c_cur (when it continues)
-        const float qom = S.qom, qs = S.qs, subk = S.subk;
-
-        // A particle of tile cell kc at offsets (ox,oy,oz) sitting in another cell b (an arrival of
-        // the lagged sort): full processing by one lane.
-        auto arrive = [&](float ox, float oy, float oz, float vx, float vy, float vz, int kc, uint32_t id) {
-            int qlx, qly, qlz;
-            G.split(kc, qlx, qly, qlz);
-            const int dbx = dcell(ox), dby = dcell(oy), dbz = dcell(oz);
-            float px = ox - (float)dbx, py = oy - (float)dby, pz = oz - (float)dbz;
-            const int blx = qlx + dbx, bly = qly + dby, blz = qlz + dbz;  // tile-local cell b
-            const int bx = x0 + blx, by = y0 + bly, bz = z0 + blz;        // unwrapped
-            const int bxw = wrapc(bx, g.n[0]), byw = wrapc(by, g.n[1]), bzw = wrapc(bz, g.n[2]);
-            bool sunk = false;
-            int dex = 0, dey = 0, dez = 0;
-            if (MODE == MODE_PUSH) {
-                float Ex, Ey, Ez, Bx, By, Bz;
-                if (DIPOLE) {
-                    Ex = Ey = Ez = 0.0f;
-                    dipole_field(g, bxw, byw, bzw, px, py, pz, Bx, By, Bz);
-                } else if ((unsigned)blx < (unsigned)G.T0 && (unsigned)bly < (unsigned)G.T1 &&
-                           (unsigned)blz < (unsigned)G.T2)
-                    gather_lds(sF4, sF2, blx * fsx + bly * fsy + blz, fsx, fsy, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
+        for (int s = sg; s < sg + ns; ++s) {
+            const SpArgs& S = A.sp[s];
+            const Rsrc rin = make_rsrc(S.in, S.cap * 24);
+            const Rsrc rout = make_rsrc(S.out, S.cap * 24);
+            const unsigned cs = (unsigned)S.cap * 4u;  // byte stride between the six arrays
+            const int* s_seg = s_segs + (s - sg) * (G.TC + 1);
+            const int* s_wlo = s_wlos + (s - sg) * (NW + 1);
+            const int chi = s_wlo[wid + 1];
+            int c_cur = s_wlo[wid];
+            int pos_cur = s_seg[c_cur];
+            int carry = 0;  // stayers already placed for cell c_cur (when it continues)
+            const float qom = S.qom, qs = S.qs, subk = S.subk;
+            // the counters of a block with fewer than 2^16 particles of the species are half words in
+            // LDS, one for each of the SPG species
+            const bool small = s_seg[s_wlo[NW]] - s_seg[s_wlo[0]] < 65536;
+            const unsigned one16 = 1u << (16 * (s - sg));
+            auto count_at = [&](int x, int y, int z) {  // one more particle in tile-local cell (x,y,z)
+                if (small && (unsigned)x < (unsigned)G.T0 && (unsigned)y < (unsigned)G.T1 && (unsigned)z < (unsigned)G.T2)
+                    atomicAdd(&s_cnt[(x * G.T1 + y) * G.T2 + z], one16);
                 else
-                    gather_direct(A, bxw, byw, bzw, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
-                boris_move(g, qom, subk, Ex, Ey, Ez, Bx, By, Bz, vx, vy, vz, px, py, pz);
-                if (REFLECT) reflect_faces(g, bxw, byw, bzw, px, py, pz, vx, vy, vz);
-                sunk = !finite3(px, py, pz);
-                if (!sunk) {
-                    dex = dcell(px); dey = dcell(py); dez = dcell(pz);
-                }
-                if (SINK && !sunk) {
-                    const float rx_ = g.origin[0] + ((float)wrapc(bx + dex, g.n[0]) + px - (float)dex) * g.w[0] - g.sink_c[0];
-                    const float ry_ = g.origin[1] + ((float)wrapc(by + dey, g.n[1]) + py - (float)dey) * g.w[1] - g.sink_c[1];
-                    const float rz_ = g.origin[2] + ((float)wrapc(bz + dez, g.n[2]) + pz - (float)dez) * g.w[2] - g.sink_c[2];
-                    sunk = (rx_ * rx_ + ry_ * ry_ + rz_ * rz_) <= g.sink_r2;
-                }
-            }
-            bool ok = true;
-            if (MODE != MODE_DEPOSIT) {
-                const int bc = G.cid(g, bxw, byw, bzw);
-                const int oidx = S.start[bc] + S.stay[bc] + atomicAdd(&S.arr[bc], 1);
-                if (oidx < 0 || oidx >= S.start[bc + 1] || (long long)oidx >= S.cap) {
-                    atomicOr(A.err, ERR_SLOT);
-                    ok = false;
-                } else {
-                    store_particle(rout, cs, oidx, sunk ? NaNf : px, py, pz, vx, vy, vz);
-                    if (TRACK) S.id_out[oidx] = id;
-                }
-            }
-            if (MODE == MODE_PUSH && sunk) {
-                atomicAdd(A.removed, 1ull);
-            } else if (MODE != MODE_REBIN && ok) {
-                float wt[8];
-                tri_weights(px - (float)dex, py - (float)dey, pz - (float)dez, wt);
-                deposit_direct(A, G, sJ, x0, y0, z0, blx + dex, bly + dey, blz + dez, wt, qs * vx, qs * vy,
-                               qs * vz);
-                if (MODE == MODE_PUSH) {
-                    count_add(g, G, s_cnt, S.cnt_acc, x0, y0, z0, bx + dex, by + dey, bz + dez);
-                    if ((dex | dey | dez) == 0) count_add(g, G, s_stay, S.stay_acc, x0, y0, z0, bx, by, bz);
-                }
-            }
-        };
-        // leavers: deposit and count at the new cell, one per lane; empties the buffer
-        int kn = 0;
-        auto drain_leavers = [&]() {
-            const int kq_n = min(kn, K0CAP);
-            for (int qi = lane; qi < kq_n; qi += WS) {
-                const float* e = K0 + qi * 7;
-                const float px = e[0], py = e[1], pz = e[2], vx = e[3], vy = e[4], vz = e[5];
-                const int kc = __float_as_int(e[6]);  // the tile cell it left
-                int qlx, qly, qlz;
-                G.split(kc, qlx, qly, qlz);
-                const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
-                float wt[8];
-                tri_weights(px - (float)dex, py - (float)dey, pz - (float)dez, wt);
-                deposit_direct(A, G, sJ, x0, y0, z0, qlx + dex, qly + dey, qlz + dez, wt, qs * vx, qs * vy, qs * vz);
-                count_add(g, G, s_cnt, S.cnt_acc, x0, y0, z0, x0 + qlx + dex, y0 + qly + dey, z0 + qlz + dez);
-            }
-            wave_sync();
-            kn = 0;
-        };
-        int qn = 0;
+                    count_in(g, G, S.cnt_acc, x0 + x, y0 + y, z0 + z);
+            };
 
-        while (c_cur < chi) {
-            // runs of the next 64 cells (lane l looks at cell c_cur + l)
-            const int cl = c_cur + lane;
-            int remp = 0;
-            if (cl < chi) remp = s_seg[cl + 1] - (lane == 0 ? pos_cur : s_seg[cl]);
-            const int rl = (remp + KRUN - 1) / KRUN;
-            const int incl = wave_incl_scan(rl, lane);
-            R[lane + 1] = incl;
-            if (lane == 0) R[0] = 0;
-            // run heads: H[r] = the cell whose first run is run r (0 elsewhere); the cell of run r
-            // is then the running maximum of H up to r
-            H[lane] = 0;
-            wave_sync();
-            if (rl > 0 && incl - rl < WS) H[incl - rl] = lane;
-            const int all_runs = __shfl(incl, WS - 1, WS);
-            wave_sync();
-            const int nruns = min(all_runs, WS);
-            if (nruns == 0) {  // the next 64 cells are empty
-                c_cur = min(c_cur + WS, chi);
-                pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
-                carry = 0;
-                continue;
-            }
-            const bool active = lane < nruns;
-            int k = wave_incl_max(H[lane]), len = 0, pst = 0;  // the run's cell: c_cur + k
-            if (active) {
-                const int j = lane - R[k];
-                const int nr = R[k + 1] - R[k];
-                const int p0 = (k == 0) ? pos_cur : s_seg[c_cur + k];
-                const int nc = s_seg[c_cur + k + 1] - p0;
-                const int bl = nc < (1 << 21) ? fdivi(nc, __builtin_amdgcn_rcpf((float)nr)) : nc / nr;
-                const int rem = nc - bl * nr;
-                len = bl + (j < rem ? 1 : 0);
-                pst = p0 + j * bl + min(j, rem);
-            }
-            const int plo = __shfl(pst, 0, WS);
-            const int phi = __shfl(pst + len, nruns - 1, WS);
-            if (plo < 0 || (long long)phi > S.cap || phi - plo > WCH || phi < plo) {  // uniform over the wave
-                if (lane == 0) atomicOr(A.err, ERR_CHUNK);
-                break;
-            }
-            // the run cell's output range [a_start, a_end), loaded with the run so that both loads
-            // are in flight together
-            const int c_run = c_cur + k;
-            const int a_start = (MODE != MODE_DEPOSIT && active) ? S.start[cbase + c_run] : 0;
-            const int a_end = (MODE != MODE_DEPOSIT && active) ? S.start[cbase + c_run + 1] : 0;
-            // this lane's run into registers
-            float rx[KRUN], ry[KRUN], rz[KRUN], rvx[KRUN], rvy[KRUN], rvz[KRUN];
-            uint32_t rid[TRACK ? KRUN : 1];
-            const unsigned vrun = (unsigned)pst * 4u;
-            {
-                // Four particles of an array in one 16-byte load and the fifth in one more: 12 load
-                // instructions a run instead of 30 (128^3 x 32: 1.157 -> 1.118 ms).  Slots past the
-                // run's end read its successors (0 past the buffer's end: the range check is per
-                // word) and are cleared; a lane without a slot points past the buffer.
-                static_assert(KRUN == 5, "a run is four particles and one more");
-                typedef unsigned u4 __attribute__((ext_vector_type(4)));
-                const unsigned v4o = len > 0 ? vrun : 0xfffffff0u, v1o = len > 4 ? vrun + 16u : 0xfffffff0u;
-                auto load = [&](float (&r)[KRUN], unsigned off) {
-                    const u4 q = __builtin_amdgcn_raw_buffer_load_b128(rin, v4o, off, 0);
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) r[jj] = __uint_as_float(q[jj]);
-                    r[4] = ldp(rin, v1o, off);
-                };
-                load(rx, 0);
-                load(ry, cs);
-                load(rz, 2 * cs);
-                load(rvx, 3 * cs);
-                load(rvy, 4 * cs);
-                load(rvz, 5 * cs);
-#pragma unroll
-                for (int jj = 0; jj < KRUN; ++jj)
-                    if (jj >= len) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
-                if (TRACK)
-#pragma unroll
-                    for (int jj = 0; jj < KRUN; ++jj) rid[jj] = jj < len ? S.id_in[pst + jj] : 0u;
-            }
-            const int c = c_run;
-            int lx, ly, lz;
-            G.split(c, lx, ly, lz);
-            const int ax = x0 + lx, ay = y0 + ly, az = z0 + lz;
-            const int nb = lx * fsx + ly * fsy + lz;  // the run cell's first node in the LDS field
-
-            // pass A: the run's home particles, bit jj of hm (particles of segment a still in cell
-            // a, the fast path; NaN: no); they are the stayers that take the cell's first slots
-            unsigned hm = 0;
-#pragma unroll
-            for (int jj = 0; jj < KRUN; ++jj)
-                if (in_cell(rx[jj], ry[jj], rz[jj])) hm |= 1u << jj;
-            hm &= (1u << len) - 1u;  // empty slots hold zeros
-            const int my_stay = (MODE != MODE_DEPOSIT) ? __popc(hm) : 0;
-            const int sincl = wave_incl_scan(my_stay, lane);
-            const int sex = sincl - my_stay;
-            const int sfirst = __shfl(sex, R[k], WS);
-            const int base = (k == 0 ? carry : 0) + sex - sfirst;
-
-            // slots of the run cell's stayers lie in [0, a_lim): below its end and the capacity
-            const int a_lim = min(a_end, (int)S.cap);  // S.cap < 2^31 (one buffer resource < 4 GiB)
-
-            // pass B1, push of the home particles in place in the run registers (gather, Boris,
-            // reflection, sink); a removed particle gets a NaN x offset.  The run cell's 8 corner
-            // nodes are read from LDS once per run and held in registers for this pass only, so
-            // they never share the register file with the deposit moments of pass B2.
-            unsigned im = hm, sm = 0;  // home particles that end the step in the run's cell; removed ones
-            if (MODE == MODE_PUSH) {
-                float4 rn4[8];
-                float2 rn2[8];
-                if (!DIPOLE) {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-#pragma unroll
-                            for (int kk = 0; kk < 2; ++kk) {
-                                const int nn = nb + i * fsx + j * fsy + kk;
-                                rn4[(i * 2 + j) * 2 + kk] = sF4[nn];
-                                rn2[(i * 2 + j) * 2 + kk] = sF2[nn];
-                            }
-                }
-#pragma unroll
-                for (int jj = 0; jj < KRUN; ++jj) {
-                    if (hm & (1u << jj)) {
-                        float px = rx[jj], py = ry[jj], pz = rz[jj];
-                        float vx = rvx[jj], vy = rvy[jj], vz = rvz[jj];
-                        float Ex, Ey, Ez, Bx, By, Bz;
-                        if (DIPOLE) {
-                            Ex = Ey = Ez = 0.0f;
-                            dipole_field(g, ax, ay, az, px, py, pz, Bx, By, Bz);
-                        } else {
-                            gather_regs(rn4, rn2, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
-                        }
-                        boris_move(g, qom, subk, Ex, Ey, Ez, Bx, By, Bz, vx, vy, vz, px, py, pz);
-                        if (REFLECT) reflect_faces(g, ax, ay, az, px, py, pz, vx, vy, vz);
-                        bool sunk = false;
-                        if (!in_cell(px, py, pz)) {
-                            im &= ~(1u << jj);
-                            sunk = !finite3(px, py, pz);
-                        }
-                        if (SINK && !sunk) {
-                            const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
-                            const float sx_ = g.origin[0] + ((float)wrapc(ax + dex, g.n[0]) + px - (float)dex) * g.w[0] - g.sink_c[0];
-                            const float sy_ = g.origin[1] + ((float)wrapc(ay + dey, g.n[1]) + py - (float)dey) * g.w[1] - g.sink_c[1];
-                            const float sz_ = g.origin[2] + ((float)wrapc(az + dez, g.n[2]) + pz - (float)dez) * g.w[2] - g.sink_c[2];
-                            sunk = (sx_ * sx_ + sy_ * sy_ + sz_ * sz_) <= g.sink_r2;
-                        }
-                        if (sunk) {
-                            sm |= 1u << jj;
-                            im &= ~(1u << jj);
-                            px = NaNf;
-                        }
-                        rx[jj] = px;
-                        ry[jj] = py;
-                        rz[jj] = pz;
-                        rvx[jj] = vx;
-                        rvy[jj] = vy;
-                        rvz[jj] = vz;
-                    }
-                }
-            }
-
-            // pass B2: slots, removal counts and deposit moments of the home particles; queue
-            // entries for the others (their registers are untouched by pass B1)
-            float mom[3][8];
-#pragma unroll
-            for (int m = 0; m < 8; ++m) mom[0][m] = mom[1][m] = mom[2][m] = 0.0f;
-            float jmax = 0.0f;  // largest |j| component of the run: bounds every corner sum / run_in
-            // this run's arrivals: particles that sit in another cell (queued by input index)
-            unsigned amask = 0;
-#pragma unroll
-            for (int jj = 0; jj < KRUN; ++jj)
-                if (!((hm >> jj) & 1u) && jj < len && alive(rx[jj], ry[jj], rz[jj])) amask |= 1u << jj;
-            const bool dead = (((1u << len) - 1u) & ~hm & ~amask) != 0u || sm != 0u;
-            // Arrivals, one of every lane that has one left, wait in the queue with all their data:
-            // read again by input index when a wave of them is there, they miss L2 and cost 0.35 of
-            // the 3.9 GB of a push at 128^3 x 32 (1.118 -> 1.083 ms).  A round that does not fit is
-            // handled at once, its idle lanes taking entries from the queue.
-            for (unsigned m = amask;;) {
-                const unsigned long long bq = __ballot(m != 0);
-                if (bq == 0) break;
-                const int jl = m ? __builtin_ctz(m) : 0, nq = __popcll(bq), rank = ballot_rank(bq);
-                float e0 = rx[0], e1 = ry[0], e2 = rz[0], e3 = rvx[0], e4 = rvy[0], e5 = rvz[0];
-                uint32_t e7 = TRACK ? rid[0] : 0u;
-#pragma unroll
-                for (int jj = 1; jj < KRUN; ++jj) {
-                    const bool at = jj == jl;
-                    e0 = at ? rx[jj] : e0; e1 = at ? ry[jj] : e1; e2 = at ? rz[jj] : e2;
-                    e3 = at ? rvx[jj] : e3; e4 = at ? rvy[jj] : e4; e5 = at ? rvz[jj] : e5;
-                    if (TRACK) e7 = at ? rid[jj] : e7;
-                }
-                bool have = m != 0;
-                if (qn + nq <= QCAP) {
-                    if (have) {
-                        float* e = Q + (qn + rank) * QW;
-                        e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
-                        e[6] = __int_as_float(c);
-                        if (TRACK) e[7] = __uint_as_float(e7);
-                    }
-                    qn += nq;
-                } else {
-                    const int from = qn - 1 - (lane - rank);  // idle lanes take the queue's last entries
-                    int kc = c;
-                    if (!have && from >= 0) {
-                        const float* e = Q + from * QW;
-                        e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
-                        kc = __float_as_int(e[6]);
-                        if (TRACK) e7 = __float_as_uint(e[7]);
-                        have = true;
-                    }
-                    if (have) arrive(e0, e1, e2, e3, e4, e5, kc, e7);
-                    qn = max(0, qn - (WS - nq));
+            // leavers: deposit and count at the new cell, one per lane; empties the buffer
+            int kn = 0;
+            auto drain_leavers = [&]() {
+                const int kq_n = min(kn, K0CAP);
+                for (int qi = lane; qi < kq_n; qi += WS) {
+                    const float* e = K0 + qi * 7;
+                    const float px = e[0], py = e[1], pz = e[2], vx = e[3], vy = e[4], vz = e[5];
+                    const int kc = __float_as_int(e[6]);  // the tile cell it left
+                    int qlx, qly, qlz;
+                    G.split(kc, qlx, qly, qlz);
+                    const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
+                    float wt[8];
+                    tri_weights(px - (float)dex, py - (float)dey, pz - (float)dez, wt);
+                    deposit_direct(A, G, sJ, x0, y0, z0, qlx + dex, qly + dey, qlz + dez, wt, qs * vx, qs * vy, qs * vz);
+                    count_at(qlx + dex, qly + dey, qlz + dez);
                 }
                 wave_sync();
-                m &= m - 1;
-            }
-            // A run with a single slot that is not home (an arrival, or a particle removed in the
-            // previous step) closes the gap: the home particles move down one register, and the
-            // run is stored like a run of home particles only.  (Not in the instances that carry particle
-            // ids, where the extra registers would spill; they store such runs particle by
-            // particle.)
-            if (MODE != MODE_DEPOSIT && !TRACK) {
-                const unsigned gap = ((1u << len) - 1u) & ~hm;
-                const bool one_gap = gap != 0u && (gap & (gap - 1u)) == 0u;
-                if (__ballot(one_gap)) {
-                    const int zg = one_gap ? __builtin_ctz(gap) : KRUN;
-#pragma unroll
-                    for (int i = 0; i + 1 < KRUN; ++i) {
-                        const bool sh = i >= zg;
-                        rx[i] = sh ? rx[i + 1] : rx[i];
-                        ry[i] = sh ? ry[i + 1] : ry[i];
-                        rz[i] = sh ? rz[i + 1] : rz[i];
-                        rvx[i] = sh ? rvx[i + 1] : rvx[i];
-                        rvy[i] = sh ? rvy[i + 1] : rvy[i];
-                        rvz[i] = sh ? rvz[i + 1] : rvz[i];
-                    }
-                    if (one_gap) {
-                        --len;
-                        hm = (1u << len) - 1u;
-                        const unsigned lo = (1u << zg) - 1u;
-                        im = (im & lo) | ((im >> 1) & ~lo);
-                        sm = (sm & lo) | ((sm >> 1) & ~lo);
-                    }
+                kn = 0;
+            };
+            int qn = 0;
+
+            while (c_cur < chi) {
+                // runs of the next 64 cells (lane l looks at cell c_cur + l)
+                const int cl = c_cur + lane;
+                int remp = 0;
+                if (cl < chi) remp = s_seg[cl + 1] - (lane == 0 ? pos_cur : s_seg[cl]);
+                const int rl = (remp + KRUN - 1) / KRUN;
+                const int incl = wave_incl_scan(rl, lane);
+                R[lane + 1] = incl;
+                if (lane == 0) R[0] = 0;
+                // run heads: H[r] = the cell whose first run is run r (0 elsewhere); the cell of run r
+                // is then the running maximum of H up to r
+                H[lane] = 0;
+                wave_sync();
+                if (rl > 0 && incl - rl < WS) H[incl - rl] = lane;
+                const int all_runs = __shfl(incl, WS - 1, WS);
+                wave_sync();
+                const int nruns = min(all_runs, WS);
+                if (nruns == 0) {  // the next 64 cells are empty
+                    c_cur = min(c_cur + WS, chi);
+                    pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
+                    carry = 0;
+                    continue;
                 }
-            }
-            // a run of home particles only (the common case) takes consecutive slots: its six
-            // arrays go out in a few stores covering whole lines across the wave
-            const bool whole = (MODE != MODE_DEPOSIT) && len > 0 && hm == (1u << len) - 1u;
-            if (whole) {
-                const int o0 = a_start + base;
-                if (o0 < 0 || o0 + len > a_lim) {
-                    atomicOr(A.err, ERR_SLOT);
-                } else {
-                    const unsigned vo = (unsigned)o0 * 4u;
-                    // the first four of each array in one dwordx4 store, the rest one by one
-                    if (KRUN >= 4 && len >= 4) {
-                        st4(rout, vo, 0, rx);
-                        st4(rout, vo, cs, ry);
-                        st4(rout, vo, 2 * cs, rz);
-                        st4(rout, vo, 3 * cs, rvx);
-                        st4(rout, vo, 4 * cs, rvy);
-                        st4(rout, vo, 5 * cs, rvz);
-                    }
-                    const int jlo = (KRUN >= 4 && len >= 4) ? 4 : 0;
+                const bool active = lane < nruns;
+                int k = wave_incl_max(H[lane]), len = 0, pst = 0;  // the run's cell: c_cur + k
+                if (active) {
+                    const int j = lane - R[k];
+                    const int nr = R[k + 1] - R[k];
+                    const int p0 = (k == 0) ? pos_cur : s_seg[c_cur + k];
+                    const int nc = s_seg[c_cur + k + 1] - p0;
+                    const int bl = nc < (1 << 21) ? fdivi(nc, __builtin_amdgcn_rcpf((float)nr)) : nc / nr;
+                    const int rem = nc - bl * nr;
+                    len = bl + (j < rem ? 1 : 0);
+                    pst = p0 + j * bl + min(j, rem);
+                }
+                const int plo = __shfl(pst, 0, WS);
+                const int phi = __shfl(pst + len, nruns - 1, WS);
+                if (plo < 0 || (long long)phi > S.cap || phi - plo > WCH || phi < plo) {  // uniform over the wave
+                    if (lane == 0) atomicOr(A.err, ERR_CHUNK);
+                    break;
+                }
+                // the run cell's output range [a_start, a_end), loaded with the run so that both loads
+                // are in flight together
+                const int c_run = c_cur + k;
+                const int a_start = (MODE != MODE_DEPOSIT && active) ? S.start[cbase + c_run] : 0;
+                const int a_end = (MODE != MODE_DEPOSIT && active) ? S.start[cbase + c_run + 1] : 0;
+                // this lane's run into registers
+                float rx[KRUN], ry[KRUN], rz[KRUN], rvx[KRUN], rvy[KRUN], rvz[KRUN];
+                uint32_t rid[TRACK ? KRUN : 1];
+                const unsigned vrun = (unsigned)pst * 4u;
+                {
+                    // Four particles of an array in one 16-byte load and the fifth in one more: 12 load
+                    // instructions a run instead of 30 (128^3 x 32: 1.157 -> 1.118 ms).  Slots past the
+                    // run's end read its successors (0 past the buffer's end: the range check is per
+                    // word) and are cleared; a lane without a slot points past the buffer.
+                    static_assert(KRUN == 5, "a run is four particles and one more");
+                    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+                    const unsigned v4o = len > 0 ? vrun : 0xfffffff0u, v1o = len > 4 ? vrun + 16u : 0xfffffff0u;
+                    auto load = [&](float (&r)[KRUN], unsigned off) {
+                        const u4 q = __builtin_amdgcn_raw_buffer_load_b128(rin, v4o, off, 0);
+#pragma unroll
+                        for (int jj = 0; jj < 4; ++jj) r[jj] = __uint_as_float(q[jj]);
+                        r[4] = ldp(rin, v1o, off);
+                    };
+                    load(rx, 0);
+                    load(ry, cs);
+                    load(rz, 2 * cs);
+                    load(rvx, 3 * cs);
+                    load(rvy, 4 * cs);
+                    load(rvz, 5 * cs);
 #pragma unroll
                     for (int jj = 0; jj < KRUN; ++jj)
-                        if (jj >= jlo && jj < len)
-                            store_particle(rout, cs, o0 + jj, rx[jj], ry[jj], rz[jj], rvx[jj], rvy[jj], rvz[jj]);
+                        if (jj >= len) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
                     if (TRACK)
 #pragma unroll
-                        for (int jj = 0; jj < KRUN; ++jj)
-                            if (jj < len) S.id_out[o0 + jj] = rid[jj];
+                        for (int jj = 0; jj < KRUN; ++jj) rid[jj] = jj < len ? S.id_in[pst + jj] : 0u;
                 }
-            }
-            if (MODE != MODE_DEPOSIT && !whole && hm) {
-                int rank = 0;
+                const int c = c_run;
+                int lx, ly, lz;
+                G.split(c, lx, ly, lz);
+                const int ax = x0 + lx, ay = y0 + ly, az = z0 + lz;
+                const int nb = lx * fsx + ly * fsy + lz;  // the run cell's first node in the LDS field
+
+                // pass A: the run's home particles, bit jj of hm (particles of segment a still in cell
+                // a, the fast path; NaN: no); they are the stayers that take the cell's first slots
+                unsigned hm = 0;
 #pragma unroll
                 for (int jj = 0; jj < KRUN; ++jj)
-                    if ((hm >> jj) & 1u) {
-                        const int oidx = a_start + base + rank;
-                        ++rank;
-                        if ((unsigned)oidx >= (unsigned)a_lim) {
-                            atomicOr(A.err, ERR_SLOT);
-                        } else {
-                            store_particle(rout, cs, oidx, rx[jj], ry[jj], rz[jj], rvx[jj], rvy[jj], rvz[jj]);
-                            if (TRACK) S.id_out[oidx] = rid[jj];
+                    if (in_cell(rx[jj], ry[jj], rz[jj])) hm |= 1u << jj;
+                hm &= (1u << len) - 1u;  // empty slots hold zeros
+                const int my_stay = (MODE != MODE_DEPOSIT) ? __popc(hm) : 0;
+                const int sincl = wave_incl_scan(my_stay, lane);
+                const int sex = sincl - my_stay;
+                const int sfirst = __shfl(sex, R[k], WS);
+                const int base = (k == 0 ? carry : 0) + sex - sfirst;
+
+                // slots of the run cell's stayers lie in [0, a_lim): below its end and the capacity
+                const int a_lim = min(a_end, (int)S.cap);  // S.cap < 2^31 (one buffer resource < 4 GiB)
+
+                // pass B1, push of the home particles in place in the run registers (gather, Boris,
+                // reflection, sink); a removed particle gets a NaN x offset.  The run cell's 8 corner
+                // nodes are read from LDS once per run and held in registers for this pass only, so
+                // they never share the register file with the deposit moments of pass B2.
+                unsigned im = hm, sm = 0;  // home particles that end the step in the run's cell; removed ones
+                if (MODE == MODE_PUSH) {
+                    float4 rn4[8];
+                    float2 rn2[8];
+                    if (!DIPOLE) {
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+#pragma unroll
+                            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                                for (int kk = 0; kk < 2; ++kk) {
+                                    const int nn = nb + i * fsx + j * fsy + kk;
+                                    rn4[(i * 2 + j) * 2 + kk] = sF4[nn];
+                                    rn2[(i * 2 + j) * 2 + kk] = sF2[nn];
+                                }
+                    }
+#pragma unroll
+                    for (int jj = 0; jj < KRUN; ++jj) {
+                        if (hm & (1u << jj)) {
+                            float px = rx[jj], py = ry[jj], pz = rz[jj];
+                            float vx = rvx[jj], vy = rvy[jj], vz = rvz[jj];
+                            float Ex, Ey, Ez, Bx, By, Bz;
+                            if (DIPOLE) {
+                                Ex = Ey = Ez = 0.0f;
+                                dipole_field(g, ax, ay, az, px, py, pz, Bx, By, Bz);
+                            } else {
+                                gather_regs(rn4, rn2, px, py, pz, Ex, Ey, Ez, Bx, By, Bz);
+                            }
+                            boris_move(g, qom, subk, Ex, Ey, Ez, Bx, By, Bz, vx, vy, vz, px, py, pz);
+                            if (REFLECT) reflect_faces(g, ax, ay, az, px, py, pz, vx, vy, vz);
+                            bool sunk = false;
+                            if (!in_cell(px, py, pz)) {
+                                im &= ~(1u << jj);
+                                sunk = !finite3(px, py, pz);
+                            }
+                            if (SINK && !sunk) {
+                                const int dex = dcell(px), dey = dcell(py), dez = dcell(pz);
+                                const float sx_ = g.origin[0] + ((float)wrapc(ax + dex, g.n[0]) + px - (float)dex) * g.w[0] - g.sink_c[0];
+                                const float sy_ = g.origin[1] + ((float)wrapc(ay + dey, g.n[1]) + py - (float)dey) * g.w[1] - g.sink_c[1];
+                                const float sz_ = g.origin[2] + ((float)wrapc(az + dez, g.n[2]) + pz - (float)dez) * g.w[2] - g.sink_c[2];
+                                sunk = (sx_ * sx_ + sy_ * sy_ + sz_ * sz_) <= g.sink_r2;
+                            }
+                            if (sunk) {
+                                sm |= 1u << jj;
+                                im &= ~(1u << jj);
+                                px = NaNf;
+                            }
+                            rx[jj] = px;
+                            ry[jj] = py;
+                            rz[jj] = pz;
+                            rvx[jj] = vx;
+                            rvy[jj] = vy;
+                            rvz[jj] = vz;
                         }
                     }
-            }
-            if (MODE == MODE_PUSH && sm) atomicAdd(A.removed, (unsigned long long)__popc(sm));
-            const unsigned lmask = (MODE == MODE_PUSH) ? hm & ~im & ~sm : 0u;  // leavers: queued below
-            const int run_in = (MODE == MODE_REBIN) ? 0 : __popc(im);
-            if (MODE != MODE_REBIN) {
-                // Moments of the particles that stay: the others add zeros through their charge.
-                // Their offsets have to be finite for that, which those of removed ones are not.
-                if (__ballot(dead)) {
-#pragma unroll
-                    for (int jj = 0; jj < KRUN; ++jj)
-                        if (!((im | lmask) >> jj & 1u)) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
                 }
+
+                // pass B2: slots, removal counts and deposit moments of the home particles; queue
+                // entries for the others (their registers are untouched by pass B1)
+                float mom[3][8];
 #pragma unroll
-                for (int jj = 0; jj < KRUN; ++jj) {
-                    const float dx = rx[jj], dy = ry[jj], dz = rz[jj];
-                    const float qj = ((im >> jj) & 1u) ? qs : 0.0f;
-                    const float jx = qj * rvx[jj], jy = qj * rvy[jj], jz = qj * rvz[jj];
-                    jmax = fmaxf(jmax, fmaxf(fabsf(jx), fmaxf(fabsf(jy), fabsf(jz))));
-                    const float xy = dx * dy, xz = dx * dz, yz = dy * dz, xyz = xy * dz;
-                    const float mono[8] = {1.0f, dx, dy, dz, xy, xz, yz, xyz};
+                for (int m = 0; m < 8; ++m) mom[0][m] = mom[1][m] = mom[2][m] = 0.0f;
+                float jmax = 0.0f;  // largest |j| component of the run: bounds every corner sum / run_in
+                // this run's arrivals: particles that sit in another cell (queued by input index)
+                unsigned amask = 0;
 #pragma unroll
-                    for (int m = 0; m < 8; ++m) {
-                        mom[0][m] = fmaf(jx, mono[m], mom[0][m]);
-                        mom[1][m] = fmaf(jy, mono[m], mom[1][m]);
-                        mom[2][m] = fmaf(jz, mono[m], mom[2][m]);
-                    }
-                }
-            }
-            // leavers, one of every lane that has one left, wait in their buffer; without room they
-            // are handled in place
-            if (MODE == MODE_PUSH)
-                for (unsigned m = lmask;;) {
-                    const unsigned long long bk = __ballot(m != 0);
-                    if (bk == 0) break;
-                    const int jl = m ? __builtin_ctz(m) : 0;
+                for (int jj = 0; jj < KRUN; ++jj)
+                    if (!((hm >> jj) & 1u) && jj < len && alive(rx[jj], ry[jj], rz[jj])) amask |= 1u << jj;
+                const bool dead = (((1u << len) - 1u) & ~hm & ~amask) != 0u || sm != 0u;
+                // Arrivals, one of every lane that has one left, wait in the queue with all their data:
+                // read again by input index when a wave of them is there, they miss L2 and cost 0.35 of
+                // the 3.9 GB of a push at 128^3 x 32 (1.118 -> 1.083 ms).  A round that does not fit is
+                // handled at once, its idle lanes taking entries from the queue.
+                for (unsigned m = amask;;) {
+                    const unsigned long long bq = __ballot(m != 0);
+                    if (bq == 0) break;
+                    const int jl = m ? __builtin_ctz(m) : 0, nq = __popcll(bq), rank = ballot_rank(bq);
                     float e0 = rx[0], e1 = ry[0], e2 = rz[0], e3 = rvx[0], e4 = rvy[0], e5 = rvz[0];
+                    uint32_t e7 = TRACK ? rid[0] : 0u;
 #pragma unroll
                     for (int jj = 1; jj < KRUN; ++jj) {
                         const bool at = jj == jl;
                         e0 = at ? rx[jj] : e0; e1 = at ? ry[jj] : e1; e2 = at ? rz[jj] : e2;
                         e3 = at ? rvx[jj] : e3; e4 = at ? rvy[jj] : e4; e5 = at ? rvz[jj] : e5;
+                        if (TRACK) e7 = at ? rid[jj] : e7;
                     }
-                    const int slot = kn + ballot_rank(bk);
-                    if (m != 0 && slot < K0CAP) {
-                        float* e = K0 + slot * 7;
-                        e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
-                        e[6] = __int_as_float(c);
-                    } else if (m != 0) {
-                        const int dex = dcell(e0), dey = dcell(e1), dez = dcell(e2);
-                        float wt[8];
-                        tri_weights(e0 - (float)dex, e1 - (float)dey, e2 - (float)dez, wt);
-                        deposit_direct(A, G, sJ, x0, y0, z0, lx + dex, ly + dey, lz + dez, wt, qs * e3, qs * e4, qs * e5);
-                        count_add(g, G, s_cnt, S.cnt_acc, x0, y0, z0, ax + dex, ay + dey, az + dez);
+                    bool have = m != 0;
+                    if (qn + nq <= QCAP) {
+                        if (have) {
+                            float* e = Q + (qn + rank) * QW;
+                            e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
+                            e[6] = __int_as_float(c);
+                            if (TRACK) e[7] = __uint_as_float(e7);
+                        }
+                        qn += nq;
+                    } else {
+                        const int from = qn - 1 - (lane - rank);  // idle lanes take the queue's last entries
+                        int kc = c;
+                        if (!have && from >= 0) {
+                            const float* e = Q + from * QW;
+                            e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
+                            kc = __float_as_int(e[6]);
+                            if (TRACK) e7 = __float_as_uint(e[7]);
+                            have = true;
+                        }
+                        if (have) arrive(S, small ? 16 * (s - sg) : -1, e0, e1, e2, e3, e4, e5, kc, e7);
+                        qn = max(0, qn - (WS - nq));
                     }
-                    kn = min(kn + (int)__popcll(bk), K0CAP);
+                    wave_sync();
                     m &= m - 1;
                 }
-            if (MODE != MODE_REBIN && run_in > 0) {
-                if (!(jmax * (float)run_in <= g.fix_lim)) atomicOr(A.err, ERR_JSAT);
+                // A run with a single slot that is not home (an arrival, or a particle removed in the
+                // previous step) closes the gap: the home particles move down one register, and the
+                // run is stored like a run of home particles only.  (Not in the instances that carry particle
+                // ids, where the extra registers would spill; they store such runs particle by
+                // particle.)
+                if (MODE != MODE_DEPOSIT && !TRACK) {
+                    const unsigned gap = ((1u << len) - 1u) & ~hm;
+                    const bool one_gap = gap != 0u && (gap & (gap - 1u)) == 0u;
+                    if (__ballot(one_gap)) {
+                        const int zg = one_gap ? __builtin_ctz(gap) : KRUN;
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    float N[8];
-                    mom_to_nodes(mom[d], N);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-#pragma unroll
-                            for (int kk = 0; kk < 2; ++kk) {
-                                const int l = ((lx + JH + i) * G.nj1 + (ly + JH + j)) * G.nj2 + (lz + JH + kk);
-                                fix_add(&sJ[d * G.NJ + l], N[(i * 2 + j) * 2 + kk], g.fix_scale);
-                            }
+                        for (int i = 0; i + 1 < KRUN; ++i) {
+                            const bool sh = i >= zg;
+                            rx[i] = sh ? rx[i + 1] : rx[i];
+                            ry[i] = sh ? ry[i + 1] : ry[i];
+                            rz[i] = sh ? rz[i + 1] : rz[i];
+                            rvx[i] = sh ? rvx[i + 1] : rvx[i];
+                            rvy[i] = sh ? rvy[i + 1] : rvy[i];
+                            rvz[i] = sh ? rvz[i + 1] : rvz[i];
+                        }
+                        if (one_gap) {
+                            --len;
+                            hm = (1u << len) - 1u;
+                            const unsigned lo = (1u << zg) - 1u;
+                            im = (im & lo) | ((im >> 1) & ~lo);
+                            sm = (sm & lo) | ((sm >> 1) & ~lo);
+                        }
+                    }
                 }
-            }
-            if (MODE == MODE_PUSH && run_in > 0) {
-                atomicAdd(&s_cnt[c], run_in);
-                atomicAdd(&s_stay[c], run_in);
-            }
-            wave_sync();
+                // a run of home particles only (the common case) takes consecutive slots: its six
+                // arrays go out in a few stores covering whole lines across the wave
+                const bool whole = (MODE != MODE_DEPOSIT) && len > 0 && hm == (1u << len) - 1u;
+                if (whole) {
+                    const int o0 = a_start + base;
+                    if (o0 < 0 || o0 + len > a_lim) {
+                        atomicOr(A.err, ERR_SLOT);
+                    } else {
+                        const unsigned vo = (unsigned)o0 * 4u;
+                        // the first four of each array in one dwordx4 store, the rest one by one
+                        if (KRUN >= 4 && len >= 4) {
+                            st4(rout, vo, 0, rx);
+                            st4(rout, vo, cs, ry);
+                            st4(rout, vo, 2 * cs, rz);
+                            st4(rout, vo, 3 * cs, rvx);
+                            st4(rout, vo, 4 * cs, rvy);
+                            st4(rout, vo, 5 * cs, rvz);
+                        }
+                        const int jlo = (KRUN >= 4 && len >= 4) ? 4 : 0;
+#pragma unroll
+                        for (int jj = 0; jj < KRUN; ++jj)
+                            if (jj >= jlo && jj < len)
+                                store_particle(rout, cs, o0 + jj, rx[jj], ry[jj], rz[jj], rvx[jj], rvy[jj], rvz[jj]);
+                        if (TRACK)
+#pragma unroll
+                            for (int jj = 0; jj < KRUN; ++jj)
+                                if (jj < len) S.id_out[o0 + jj] = rid[jj];
+                    }
+                }
+                if (MODE != MODE_DEPOSIT && !whole && hm) {
+                    int rank = 0;
+#pragma unroll
+                    for (int jj = 0; jj < KRUN; ++jj)
+                        if ((hm >> jj) & 1u) {
+                            const int oidx = a_start + base + rank;
+                            ++rank;
+                            if ((unsigned)oidx >= (unsigned)a_lim) {
+                                atomicOr(A.err, ERR_SLOT);
+                            } else {
+                                store_particle(rout, cs, oidx, rx[jj], ry[jj], rz[jj], rvx[jj], rvy[jj], rvz[jj]);
+                                if (TRACK) S.id_out[oidx] = rid[jj];
+                            }
+                        }
+                }
+                if (MODE == MODE_PUSH && sm) atomicAdd(A.removed, (unsigned long long)__popc(sm));
+                const unsigned lmask = (MODE == MODE_PUSH) ? hm & ~im & ~sm : 0u;  // leavers: queued below
+                const int run_in = (MODE == MODE_REBIN) ? 0 : __popc(im);
+                if (MODE != MODE_REBIN) {
+                    // Moments of the particles that stay: the others add zeros through their charge.
+                    // Their offsets have to be finite for that, which those of removed ones are not.
+                    if (__ballot(dead)) {
+#pragma unroll
+                        for (int jj = 0; jj < KRUN; ++jj)
+                            if (!((im | lmask) >> jj & 1u)) rx[jj] = ry[jj] = rz[jj] = rvx[jj] = rvy[jj] = rvz[jj] = 0.0f;
+                    }
+#pragma unroll
+                    for (int jj = 0; jj < KRUN; ++jj) {
+                        const float dx = rx[jj], dy = ry[jj], dz = rz[jj];
+                        const float qj = ((im >> jj) & 1u) ? qs : 0.0f;
+                        const float jx = qj * rvx[jj], jy = qj * rvy[jj], jz = qj * rvz[jj];
+                        jmax = fmaxf(jmax, fmaxf(fabsf(jx), fmaxf(fabsf(jy), fabsf(jz))));
+                        const float xy = dx * dy, xz = dx * dz, yz = dy * dz, xyz = xy * dz;
+                        const float mono[8] = {1.0f, dx, dy, dz, xy, xz, yz, xyz};
+#pragma unroll
+                        for (int m = 0; m < 8; ++m) {
+                            mom[0][m] = fmaf(jx, mono[m], mom[0][m]);
+                            mom[1][m] = fmaf(jy, mono[m], mom[1][m]);
+                            mom[2][m] = fmaf(jz, mono[m], mom[2][m]);
+                        }
+                    }
+                }
+                // leavers, one of every lane that has one left, wait in their buffer; without room they
+                // are handled in place
+                if (MODE == MODE_PUSH)
+                    for (unsigned m = lmask;;) {
+                        const unsigned long long bk = __ballot(m != 0);
+                        if (bk == 0) break;
+                        const int jl = m ? __builtin_ctz(m) : 0;
+                        float e0 = rx[0], e1 = ry[0], e2 = rz[0], e3 = rvx[0], e4 = rvy[0], e5 = rvz[0];
+#pragma unroll
+                        for (int jj = 1; jj < KRUN; ++jj) {
+                            const bool at = jj == jl;
+                            e0 = at ? rx[jj] : e0; e1 = at ? ry[jj] : e1; e2 = at ? rz[jj] : e2;
+                            e3 = at ? rvx[jj] : e3; e4 = at ? rvy[jj] : e4; e5 = at ? rvz[jj] : e5;
+                        }
+                        const int slot = kn + ballot_rank(bk);
+                        if (m != 0 && slot < K0CAP) {
+                            float* e = K0 + slot * 7;
+                            e[0] = e0; e[1] = e1; e[2] = e2; e[3] = e3; e[4] = e4; e[5] = e5;
+                            e[6] = __int_as_float(c);
+                        } else if (m != 0) {
+                            const int dex = dcell(e0), dey = dcell(e1), dez = dcell(e2);
+                            float wt[8];
+                            tri_weights(e0 - (float)dex, e1 - (float)dey, e2 - (float)dez, wt);
+                            deposit_direct(A, G, sJ, x0, y0, z0, lx + dex, ly + dey, lz + dez, wt, qs * e3, qs * e4, qs * e5);
+                            count_at(lx + dex, ly + dey, lz + dez);
+                        }
+                        kn = min(kn + (int)__popcll(bk), K0CAP);
+                        m &= m - 1;
+                    }
+                if (MODE != MODE_REBIN && run_in > 0) {
+                    if (!(jmax * (float)run_in <= g.fix_lim)) atomicOr(A.err, ERR_JSAT);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        float N[8];
+                        mom_to_nodes(mom[d], N);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+#pragma unroll
+                            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                                for (int kk = 0; kk < 2; ++kk) {
+                                    const int l = ((lx + JH + i) * G.nj1 + (ly + JH + j)) * G.nj2 + (lz + JH + kk);
+                                    fix_add(&sJ[d * G.NJ + l], N[(i * 2 + j) * 2 + kk], g.fix_scale);
+                                }
+                    }
+                }
+                if (MODE == MODE_PUSH && run_in > 0) {
+                    // (a cell's half word holds its stayers also in a larger block, unless it is a
+                    // very large cell)
+                    if (s_seg[c + 1] - s_seg[c] < 32768) {
+                        atomicAdd(&s_stay[c], run_in * one16);
+                    } else {
+                        atomicAdd(&S.stay_acc[cbase + c], run_in);
+                        atomicAdd(&S.cnt_acc[cbase + c], run_in);
+                    }
+                }
+                wave_sync();
 
-            // leavers wait in their buffer until it is half full
-            if (kn >= K0CAP / 2) drain_leavers();
-            // advance the wave's cursor past the runs of this chunk
-            const int klast = __shfl(k, nruns - 1, WS);
-            if (all_runs <= WS) {
-                c_cur = min(c_cur + WS, chi);
-                pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
-                carry = 0;
-            } else if (R[klast + 1] == WS) {  // the last cell ended with run 63
-                c_cur = c_cur + klast + 1;
-                pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
-                carry = 0;
-            } else {  // cell c_cur + klast continues in the next chunk
-                const int sl = __shfl(sincl, nruns - 1, WS);
-                const int s0 = __shfl(sex, R[klast], WS);
-                carry = (klast == 0 ? carry : 0) + sl - s0;
-                c_cur = c_cur + klast;
-                pos_cur = phi;
+                // leavers wait in their buffer until it is half full
+                if (kn >= K0CAP / 2) drain_leavers();
+                // advance the wave's cursor past the runs of this chunk
+                const int klast = __shfl(k, nruns - 1, WS);
+                if (all_runs <= WS) {
+                    c_cur = min(c_cur + WS, chi);
+                    pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
+                    carry = 0;
+                } else if (R[klast + 1] == WS) {  // the last cell ended with run 63
+                    c_cur = c_cur + klast + 1;
+                    pos_cur = c_cur < chi ? s_seg[c_cur] : 0;
+                    carry = 0;
+                } else {  // cell c_cur + klast continues in the next chunk
+                    const int sl = __shfl(sincl, nruns - 1, WS);
+                    const int s0 = __shfl(sex, R[klast], WS);
+                    carry = (klast == 0 ? carry : 0) + sl - s0;
+                    c_cur = c_cur + klast;
+                    pos_cur = phi;
+                }
+                wave_sync();
+            }
+            if (kn > 0) drain_leavers();  // the leavers still queued
+            if (lane < qn) {  // and the arrivals
+                const float* e = Q + lane * QW;
+                arrive(S, small ? 16 * (s - sg) : -1, e[0], e[1], e[2], e[3], e[4], e[5], __float_as_int(e[6]),
+                       TRACK ? __float_as_uint(e[QW - 1]) : 0u);
             }
             wave_sync();
         }
-        if (kn > 0) drain_leavers();  // the leavers and arrivals still queued
-        if (lane < qn) {
-            const float* e = Q + lane * QW;
-            arrive(e[0], e[1], e[2], e[3], e[4], e[5], __float_as_int(e[6]), TRACK ? __float_as_uint(e[QW - 1]) : 0u);
-        }
-        __syncthreads();
         if (MODE == MODE_PUSH) {
+            __syncthreads();
             for (int i = tid; i < G.TC; i += NTP) {
-                if (s_cnt[i]) atomicAdd(&S.cnt_acc[cbase + i], s_cnt[i]);
-                if (s_stay[i]) atomicAdd(&S.stay_acc[cbase + i], s_stay[i]);
+                const unsigned v = s_stay[i], u = s_cnt[i];
+                const int n0 = v & 0xffffu, n1 = v >> 16, m0 = n0 + (int)(u & 0xffffu), m1 = n1 + (int)(u >> 16);
+                if (n0) atomicAdd(&A.sp[sg].stay_acc[cbase + i], n0);
+                if (m0) atomicAdd(&A.sp[sg].cnt_acc[cbase + i], m0);
+                if (n1) atomicAdd(&A.sp[sg + 1].stay_acc[cbase + i], n1);
+                if (m1) atomicAdd(&A.sp[sg + 1].cnt_acc[cbase + i], m1);
             }
         }
     }
@@ -1486,12 +1520,12 @@ __global__ __launch_bounds__(NT) void k_scan_tiles(ScanArgs A) {
 // Launch order of the particle kernel's tiles for the layout the scans just produced.  A
 // block's time grows with its tile's particles.  With an uneven load (the heaviest tile more
 // than 25 % above the mean) the heaviest tiles go first (longest-processing-time order over 256
-// load classes), so that the blocks that start last are light.  Otherwise the tiles go in a
-// scrambled order, tile (b * mul) mod ntiles for block b with mul coprime to ntiles: neighbouring
-// tiles then run at different times, which on the uniform 128^3 x 32 workload takes 2 % off the
-// push against launching neighbours together (the XCD-aware order).  Any permutation gives the
-// same results: the order only schedules.
-__device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul) {
+// load classes), so that the blocks that start last are light.  Otherwise tile b goes to block b:
+// neighbouring tiles run at the same time on different XCDs (blocks are dealt round-robin over the
+// 8 XCDs).  Scrambled over the grid the push took 1.3 % more at 128^3 x 32 and 4 % more at
+// 96^3 x 32, an eighth of the grid for each XCD in turn 2 % more.  Any permutation gives the same
+// results: the order only schedules.
+__device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
     const Geo& g = A.g;
     __shared__ unsigned long long s_sum[NT / 64];
     __shared__ int s_max[NT / 64], s_w4[NT / 64];
@@ -1528,7 +1562,7 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul
         mx = max(mx, s_max[w]);
     }
     if ((double)mx * g.ntiles <= 1.25 * (double)sum || mx == 0) {
-        for (int b = tid; b < g.ntiles; b += NT) order[b] = (int)(((long long)b * mul) % g.ntiles);
+        for (int b = tid; b < g.ntiles; b += NT) order[b] = b;
         return;
     }
     auto cls = [&](int v) { return 255 - (int)(((long long)v * 255) / mx); };  // heaviest: class 0
@@ -1548,10 +1582,10 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order, int mul
 // counters are cleared for the next pass.  Every block adds up the totals of the tiles before its
 // own (16 KB at most from L2 at 128^3): a launch for the bases alone costs more than these reads.
 // A further block orders the tiles for the next push meanwhile.
-__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order, int mul) {
+__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order) {
     const Geo& g = A.g;
     if ((int)blockIdx.x == g.ntiles) {
-        if (blockIdx.y == 0) tile_order_block(A, nsp, order, mul);
+        if (blockIdx.y == 0) tile_order_block(A, nsp, order);
         return;
     }
     const ScanSp& S = A.sp[blockIdx.y];
@@ -2090,7 +2124,6 @@ struct ipic_ctx {
     unsigned long long* removed = nullptr;
     int* derr = nullptr;
     int* tile_order = nullptr;     // launch order of the particle kernel's tiles
-    int order_mul = 1;             // multiplier of the scrambled tile order, coprime to ntiles
     bool order_valid = false;      // tile_order describes the current layout's loads
     double* red = nullptr;
     int red_blocks = 1024;
@@ -2318,8 +2351,7 @@ int launch_scan(ipic_ctx* ctx) {
         hipLaunchKernelGGL(k_scan_small, dim3(ns), dim3(1024), 0, ctx->stream, A);
     } else {
         hipLaunchKernelGGL(k_scan_tiles, dim3(ctx->g.ntiles, ns), dim3(NT), 0, ctx->stream, A);
-        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order,
-                           ctx->order_mul);
+        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order);
     }
     HIPCK(ctx, hipGetLastError());
     for (int s = 0; s < ns; ++s) {  // the roles k_scan_cells gave the arrays
@@ -2846,22 +2878,6 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         if (build_jpairs(g, jp) != 0) {
             delete ctx;
             return fail(nullptr, IPIC_E_ARG, "tile/grid combination not supported");
-        }
-        {
-            // multiplier of the scrambled tile order: near 0.618 ntiles, so that consecutive
-            // blocks take tiles far apart, and coprime to ntiles, so that b -> b * mul mod
-            // ntiles is a permutation
-            auto gcd = [](int a, int b) {
-                while (b) {
-                    const int r = a % b;
-                    a = b;
-                    b = r;
-                }
-                return a;
-            };
-            int m = std::max(1, (int)(0.6180339887 * g.ntiles));
-            while (gcd(m, g.ntiles) != 1) ++m;
-            ctx->order_mul = m;
         }
         hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
         if (e != hipSuccess) {
