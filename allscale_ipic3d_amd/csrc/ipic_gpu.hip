@@ -1462,6 +1462,163 @@ __global__ __launch_bounds__(256) void k_field_B(FieldArgs F) {
     F.Bc[i] = b;
 }
 
+// K substeps of the leapfrog (or of the forward solver) and, with `last`, interpC2N, in one launch.
+// A substep is E += dt (eF curl- Bc - J) (field.h:359-363), then Bc -= dt bF curl+ E
+// (field.h:366-371).  A block loads the Bc of its LEAP_T^3 box and of the layers around it that the
+// K substeps and interpC2N reach (K + 1 below, K above) into LDS, advances E and Bc there, one
+// layer less on each side per substep, and stores its box to the other buffers, as other blocks
+// read the old values meanwhile.
+//
+// Bound: the two passes of a substep and interpC2N each read and wrote their arrays and waited for
+// a launch; here the fields move once per K substeps, and a launch is bound by the chain of its
+// phases (load, E, Bc, E, Bc, store).  Hence K = 2 and small boxes of many waves: 8 substeps and
+// interpC2N take 53 us at 64^3 (in passes 80-90) and 214 at 128^3 (378); 256 threads a
+// box of 8x8x8 62 and 271, boxes of 4x4x16 58 and 268, of 8x8x16 52 and 198, but 43 against 38.5 on
+// grids of up to 32^3; K = 4 61 and 386 (a box of 8 then computes 8 times its volume).
+constexpr int LEAP_T = 8, LEAP_THREADS = 512;
+
+struct LeapArgs {
+    Geo g;
+    const float4 *E, *B, *J;          // the state (perturbations) and the current
+    const float4 *SE, *SB, *Ebg, *Bnbg;  // static sources and background (nullable)
+    float4 *Eo, *Bo;                  // the state after the substeps
+    float4 *Eg, *Bn;                  // gather fields, written with `last`
+    float dt, eF, bF;
+    int last;
+};
+
+template <int K>
+__global__ __launch_bounds__(LEAP_THREADS) void k_leap(LeapArgs A) {
+    constexpr int TX = LEAP_T, TY = LEAP_T, TZ = LEAP_T;
+    constexpr int EX = TX + 2 * K, EY = TY + 2 * K, EZ = TZ + 2 * K, EN = EX * EY * EZ;  // E: K layers around the box
+    constexpr int BX = EX + 1, BY = EY + 1, BZ = EZ + 1, BN = BX * BY * BZ;              // Bc: one more below
+    __shared__ float sE[3][EN], sB[3][BN];
+    __shared__ int s_x[BX], s_y[BY], s_z[BZ];  // periodic offsets of Bc's layers
+    const Geo& g = A.g;
+    const int tid = threadIdx.x;
+    const int nbz = (g.n[2] + TZ - 1) / TZ, nby = (g.n[1] + TY - 1) / TY;
+    // consecutive boxes to one XCD (blocks are dealt round-robin over the 8 XCDs): their layers
+    // meet in its L2
+    const int nb = gridDim.x, per = nb / 8, rem = nb % 8, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int bb = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+    const int x0 = bb / (nby * nbz) * TX, y0 = (bb / nbz) % nby * TY, z0 = bb % nbz * TZ;
+    if (tid < BX) s_x[tid] = wrapc(x0 + tid - K - 1, g.n[0]) * g.s0;
+    if (tid < BY) s_y[tid] = wrapc(y0 + tid - K - 1, g.n[1]) * g.n[2];
+    if (tid < BZ) s_z[tid] = wrapc(z0 + tid - K - 1, g.n[2]);
+    __syncthreads();
+    auto node = [&](int i, int j, int k) { return s_x[i] + s_y[j] + s_z[k]; };  // of Bc's layers
+#pragma unroll 4
+    for (int q = tid; q < BN; q += LEAP_THREADS) {
+        const int i = q / (BY * BZ), r = q - i * (BY * BZ), j = r / BZ, k = r - j * BZ;
+        const float4 b = A.B[node(i, j, k)];
+        sB[0][q] = b.x;
+        sB[1][q] = b.y;
+        sB[2][q] = b.z;
+    }
+    const float iw0 = g.inv_w[0], iw1 = g.inv_w[1], iw2 = g.inv_w[2], dt = A.dt, c2 = A.eF, dtb = A.dt * A.bF;
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+        __syncthreads();
+        {
+            const int LX = EX - 2 * s, LY = EY - 2 * s, LZ = EZ - 2 * s;
+#pragma unroll 4
+            for (int q = tid; q < LX * LY * LZ; q += LEAP_THREADS) {
+                const int i = q / (LY * LZ) + s, r = q % (LY * LZ), j = r / LZ + s, k = r % LZ + s;
+                const int nd = node(i + 1, j + 1, k + 1), el = (i * EY + j) * EZ + k;
+                const int bl = ((i + 1) * BY + j + 1) * BZ + k + 1;
+                float4 e;
+                if (s == 0) {
+                    e = A.E[nd];
+                } else {
+                    e.x = sE[0][el];
+                    e.y = sE[1][el];
+                    e.z = sE[2][el];
+                }
+                const float4 J = A.J[nd];
+                const float bx = sB[0][bl], by = sB[1][bl], bz = sB[2][bl];
+                const float bmxy = sB[1][bl - BY * BZ], bmxz = sB[2][bl - BY * BZ];
+                const float bmyx = sB[0][bl - BZ], bmyz = sB[2][bl - BZ];
+                const float bmzx = sB[0][bl - 1], bmzy = sB[1][bl - 1];
+                e.x = e.x + dt * (c2 * ((bz - bmyz) * iw1 - (by - bmzy) * iw2) - J.x);
+                e.y = e.y + dt * (c2 * ((bx - bmzx) * iw2 - (bz - bmxz) * iw0) - J.y);
+                e.z = e.z + dt * (c2 * ((by - bmxy) * iw0 - (bx - bmyx) * iw1) - J.z);
+                if (A.SE) {
+                    const float4 se = A.SE[nd];
+                    e.x += dt * se.x;
+                    e.y += dt * se.y;
+                    e.z += dt * se.z;
+                }
+                sE[0][el] = e.x;
+                sE[1][el] = e.y;
+                sE[2][el] = e.z;
+                const int ix = i - K, iy = j - K, iz = k - K;
+                if (s == K - 1 && (unsigned)ix < (unsigned)TX && (unsigned)iy < (unsigned)TY && (unsigned)iz < (unsigned)TZ &&
+                    x0 + ix < g.n[0] && y0 + iy < g.n[1] && z0 + iz < g.n[2]) {
+                    A.Eo[nd] = make_float4(e.x, e.y, e.z, 0.0f);
+                    if (A.last && A.Eg) {
+                        const float4 eb = A.Ebg[nd];
+                        A.Eg[nd] = make_float4(e.x + eb.x, e.y + eb.y, e.z + eb.z, 0.0f);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        {
+            const int LX = BX - 2 - 2 * s, LY = BY - 2 - 2 * s, LZ = BZ - 2 - 2 * s;
+#pragma unroll 4
+            for (int q = tid; q < LX * LY * LZ; q += LEAP_THREADS) {
+                const int i = q / (LY * LZ) + s + 1, r = q % (LY * LZ), j = r / LZ + s + 1, k = r % LZ + s + 1;
+                const int bl = (i * BY + j) * BZ + k, el = ((i - 1) * EY + j - 1) * EZ + k - 1;
+                const float ex = sE[0][el], ey = sE[1][el], ez = sE[2][el];
+                const float epxy = sE[1][el + EY * EZ], epxz = sE[2][el + EY * EZ];
+                const float epyx = sE[0][el + EZ], epyz = sE[2][el + EZ];
+                const float epzx = sE[0][el + 1], epzy = sE[1][el + 1];
+                float bx = sB[0][bl], by = sB[1][bl], bz = sB[2][bl];
+                bx = bx - dtb * ((epyz - ez) * iw1 - (epzy - ey) * iw2);
+                by = by - dtb * ((epzx - ex) * iw2 - (epxz - ez) * iw0);
+                bz = bz - dtb * ((epxy - ey) * iw0 - (epyx - ex) * iw1);
+                if (A.SB) {  // the source already carries the B-pass factor
+                    const float4 sb = A.SB[node(i, j, k)];
+                    bx -= dt * sb.x;
+                    by -= dt * sb.y;
+                    bz -= dt * sb.z;
+                }
+                sB[0][bl] = bx;
+                sB[1][bl] = by;
+                sB[2][bl] = bz;
+            }
+        }
+    }
+    __syncthreads();
+    for (int q = tid; q < TX * TY * TZ; q += LEAP_THREADS) {
+        const int ix = q / (TY * TZ), r = q % (TY * TZ), iy = r / TZ, iz = r % TZ;
+        if (x0 + ix >= g.n[0] || y0 + iy >= g.n[1] || z0 + iz >= g.n[2]) continue;
+        const int i = ix + K + 1, j = iy + K + 1, k = iz + K + 1, bl = (i * BY + j) * BZ + k, nd = node(i, j, k);
+        A.Bo[nd] = make_float4(sB[0][bl], sB[1][bl], sB[2][bl], 0.0f);
+        if (!A.last) continue;
+        float sx = 0, sy = 0, sz = 0;  // in k_c2n's order
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int m = bl - a * BY * BZ - b * BZ - c;
+                    sx += sB[0][m];
+                    sy += sB[1][m];
+                    sz += sB[2][m];
+                }
+        float4 o = make_float4(0.125f * sx, 0.125f * sy, 0.125f * sz, 0.0f);
+        if (A.Bnbg) {
+            const float4 bg = A.Bnbg[nd];
+            o.x += bg.x;
+            o.y += bg.y;
+            o.z += bg.z;
+        }
+        A.Bn[nd] = o;
+    }
+}
+
 // interpC2N (field.h:234-247): node B = 1/8 sum of the 8 surrounding centres.
 __global__ __launch_bounds__(256) void k_c2n(FieldArgs F) {
     const Geo& g = F.g;
@@ -2136,6 +2293,8 @@ struct ipic_ctx {
     hipStream_t stream = nullptr;
     float4* E = nullptr;
     float4* Bc = nullptr;
+    float4* E2 = nullptr;          // what k_leap writes, swapped with E and Bc (field_substeps > 1)
+    float4* Bc2 = nullptr;
     float4* Bn = nullptr;
     float4* J = nullptr;
     float4* Eg = nullptr;     // optional device arrays of the background split
@@ -2427,23 +2586,56 @@ int slice_sum(ipic_ctx* ctx, FieldArgs& F) {
     return 0;
 }
 
-int launch_leapfrog(ipic_ctx* ctx) {
+template <int K>
+void launch_leap(ipic_ctx* ctx, int last) {
+    const FieldArgs F = field_args(ctx);
+    const LeapArgs A{ctx->g, ctx->E, ctx->Bc, ctx->J, F.SE, F.SB, F.Ebg, F.Bnbg, ctx->E2, ctx->Bc2, F.Eg, F.Bn,
+                     F.dt, F.eF, F.bF, last};
+    int nb = 1;
+    for (int k = 0; k < 3; ++k) nb *= (ctx->g.n[k] + LEAP_T - 1) / LEAP_T;
+    hipLaunchKernelGGL(k_leap<K>, dim3(nb), dim3(LEAP_THREADS), 0, ctx->stream, A);
+    std::swap(ctx->E, ctx->E2);
+    std::swap(ctx->Bc, ctx->Bc2);
+}
+
+int launch_c2n(ipic_ctx* ctx);
+int launch_jsum(ipic_ctx* ctx);
+
+// The field substeps with J held fixed, and with node_b the gather's node B.
+int launch_leapfrog(ipic_ctx* ctx, bool node_b) {
     // the static field uses no J: it is formed on demand (download, conservation, field state)
     // from the current deposit, and the next deposit pass clears the overflow accumulator
-    if (ctx->d.field_substeps == 0) return 0;
+    const int n = ctx->d.field_substeps;
+    if (n == 0) return 0;
+    if (n > 1) {
+        // Two substeps a launch.  A launch swaps the buffers, and the arrays that ipic_gpu_field_state
+        // hands out must stay the live ones: the number of launches is even, with 1 to 3 substeps
+        // in launches of their own for that (64^3, 3 substeps: 28.6 us, in passes 39).
+        int single = n % 2;
+        if ((n / 2 + single) % 2) single += 2;
+        if (int rc = launch_jsum(ctx)) return rc;
+        for (int left = n; left > 0;) {
+            const int k = left > single ? 2 : 1;
+            left -= k;
+            const int last = node_b && left == 0;
+            if (k == 2) launch_leap<2>(ctx, last);
+            else launch_leap<1>(ctx, last);
+        }
+        HIPCK(ctx, hipGetLastError());
+        return 0;
+    }
+    // One substep: the passes work in place, and the E pass forms J from the partials unless that was
+    // done already.  (128^3 with 32 particles a cell: field phase 128 us, k_jsum and k_leap<1> 138.)
     FieldArgs F = field_args(ctx);
     const int nb = (ctx->g.ncell + 255) / 256;
-    for (int s = 0; s < ctx->d.field_substeps; ++s) {
-        // the first E pass forms J from the partials unless that was done already
-        const int from_partials = (s == 0 && !ctx->j_summed) ? 1 : 0;
-        if (from_partials)
-            if (int rc = slice_sum(ctx, F)) return rc;
-        hipLaunchKernelGGL(k_field_E, dim3(nb), dim3(256), 0, ctx->stream, F, from_partials);
-        hipLaunchKernelGGL(k_field_B, dim3(nb), dim3(256), 0, ctx->stream, F);
-    }
+    const int from_partials = ctx->j_summed ? 0 : 1;
+    if (from_partials)
+        if (int rc = slice_sum(ctx, F)) return rc;
+    hipLaunchKernelGGL(k_field_E, dim3(nb), dim3(256), 0, ctx->stream, F, from_partials);
+    hipLaunchKernelGGL(k_field_B, dim3(nb), dim3(256), 0, ctx->stream, F);
     HIPCK(ctx, hipGetLastError());
     ctx->j_summed = true;
-    return 0;
+    return node_b ? launch_c2n(ctx) : 0;
 }
 
 int launch_c2n(ipic_ctx* ctx) {
@@ -2527,7 +2719,7 @@ int operator_phase(ipic_ctx* ctx, ipic_step_stats* st) {
     if (!ok) {
         if (int rc = copy_f4(ctx, ctx->E, ctx->Eb)) return rc;
         if (int rc = copy_f4(ctx, ctx->Bc, ctx->Bb)) return rc;
-        if (int rc = launch_leapfrog(ctx)) return rc;
+        if (int rc = launch_leapfrog(ctx, false)) return rc;
         if (st) st->fallback_steps++;
         return 0;
     }
@@ -2536,7 +2728,7 @@ int operator_phase(ipic_ctx* ctx, ipic_step_stats* st) {
         if (int rc = copy_f4(ctx, ctx->Bo, ctx->Bc)) return rc;
         if (int rc = copy_f4(ctx, ctx->E, ctx->Eb)) return rc;
         if (int rc = copy_f4(ctx, ctx->Bc, ctx->Bb)) return rc;
-        if (int rc = launch_leapfrog(ctx)) return rc;
+        if (int rc = launch_leapfrog(ctx, false)) return rc;
         hipLaunchKernelGGL(k_audit, dim3(ctx->red_blocks), dim3(256), 0, ctx->stream, g, F.c2, ctx->Eo, ctx->Bo,
                            ctx->E, ctx->Bc, ctx->Eb, ctx->Bb, ctx->red);
         HIPCK(ctx, hipGetLastError());
@@ -2595,12 +2787,11 @@ int field_phase(ipic_ctx* ctx, bool use_op, ipic_step_stats* st) {
     if (timing) HIPCK(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
     if (use_op && ctx->op_on) {
         if (int rc = operator_phase(ctx, st)) return rc;
-    } else {
-        if (int rc = launch_leapfrog(ctx)) return rc;
-    }
-    // a static field keeps the node B that the upload formed
-    if (ctx->d.field_substeps > 0)
         if (int rc = launch_c2n(ctx)) return rc;
+    } else {
+        // with interpC2N in its last launch; a static field keeps the node B that the upload formed
+        if (int rc = launch_leapfrog(ctx, true)) return rc;
+    }
     if (timing) {
         HIPCK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
         if (st) st->ms_field += ev_ms(ctx, 2, 3);
@@ -2956,6 +3147,10 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         const size_t nc = (size_t)g.ncell;
         rc = rc ? rc : dalloc(ctx, &ctx->E, nc);
         rc = rc ? rc : dalloc(ctx, &ctx->Bc, nc);
+        if (d.field_substeps > 1) {
+            rc = rc ? rc : dalloc(ctx, &ctx->E2, nc);
+            rc = rc ? rc : dalloc(ctx, &ctx->Bc2, nc);
+        }
         rc = rc ? rc : dalloc(ctx, &ctx->Bn, nc);
         rc = rc ? rc : dalloc(ctx, &ctx->J, nc);
         rc = rc ? rc : dalloc(ctx, &ctx->jpart, (size_t)g.ntiles * g.nsl * 3 * g.NJ);
