@@ -65,9 +65,9 @@ enum { MODE_PUSH = 0, MODE_DEPOSIT = 1, MODE_REBIN = 2 };
 
 struct Geo {
     int n[3];
-    int T[3];
+    int T[3];             // tile edges; the last tile of an axis ends with the grid and may be shorter
     int NTl[3];
-    int TC;
+    int TC;               // cells, J nodes (NJ, nj) of a full tile
     int ntiles;
     int nsl;              // blocks per tile of the particle kernel (slices of the tile's cells)
     int ncell;
@@ -92,7 +92,6 @@ struct Geo {
     float E0[3];          // uniform part of the background field (added in the gather)
     float B0[3];
     float inv_T[3];       // 1 / T (exact small-integer division by a float reciprocal)
-    float inv_T12;        // 1 / (T[1] * T[2])
     float fix_lim;        // 2^(50 - fix_bits): J in fixed point with fix_bits fractional bits
     double fix_scale;     // 2^fix_bits
     double fix_inv;       // 2^-fix_bits
@@ -159,10 +158,45 @@ __device__ __forceinline__ int wrapc(int i, int n) {
 // the quotient is offset by 0.5/b, more than the error (a + 0.5) * 2^-22 / b of the product.
 __device__ __forceinline__ int fdivi(int a, float inv_b) { return (int)(((float)a + 0.5f) * inv_b); }
 
+// The cells are numbered tile by tile (z fastest), row-major within a tile.  Tile t starts at cell
+// (x0,y0,z0), has w0 x w1 x w2 cells, and the number of its first cell is what lies before it: whole
+// layers of tiles along x, rows of tiles in its layer, tiles in its row.
+struct TileBox {
+    int x0, y0, z0, w0, w1, w2;
+    __host__ __device__ __forceinline__ int cells() const { return w0 * w1 * w2; }
+    __host__ __device__ __forceinline__ int first(const Geo& g) const {
+        return x0 * g.s0 + w0 * (y0 * g.n[2] + w1 * z0);
+    }
+};
+
+__host__ __device__ __forceinline__ TileBox tile_at(const Geo& g, int tx, int ty, int tz) {
+    const int x0 = tx * g.T[0], y0 = ty * g.T[1], z0 = tz * g.T[2];
+    const int r0 = g.n[0] - x0, r1 = g.n[1] - y0, r2 = g.n[2] - z0;
+    return {x0, y0, z0, r0 < g.T[0] ? r0 : g.T[0], r1 < g.T[1] ? r1 : g.T[1], r2 < g.T[2] ? r2 : g.T[2]};
+}
+
+__host__ __device__ __forceinline__ TileBox tile_box(const Geo& g, int t) {
+    const int q = t / g.NTl[2], tx = q / g.NTl[1];
+    return tile_at(g, tx, q - tx * g.NTl[1], t - q * g.NTl[2]);
+}
+
 __device__ __forceinline__ int cid_of(const Geo& g, int x, int y, int z) {
-    const int tx = fdivi(x, g.inv_T[0]), ty = fdivi(y, g.inv_T[1]), tz = fdivi(z, g.inv_T[2]);
-    const int lx = x - tx * g.T[0], ly = y - ty * g.T[1], lz = z - tz * g.T[2];
-    return ((tx * g.NTl[1] + ty) * g.NTl[2] + tz) * g.TC + (lx * g.T[1] + ly) * g.T[2] + lz;
+    const TileBox b = tile_at(g, fdivi(x, g.inv_T[0]), fdivi(y, g.inv_T[1]), fdivi(z, g.inv_T[2]));
+    return b.first(g) + ((x - b.x0) * b.w1 + (y - b.y0)) * b.w2 + z - b.z0;
+}
+
+// the cell of a number
+__host__ __device__ __forceinline__ void cell_of(const Geo& g, int cid, int& x, int& y, int& z) {
+    const int tx = cid / (g.T[0] * g.s0);  // every layer of tiles before the last is T[0] thick
+    int r = cid - tx * g.T[0] * g.s0;
+    const int w0 = tile_at(g, tx, 0, 0).w0, ty = r / (w0 * g.T[1] * g.n[2]);
+    r -= ty * w0 * g.T[1] * g.n[2];
+    const int w1 = tile_at(g, tx, ty, 0).w1, tz = r / (w0 * w1 * g.T[2]);
+    r -= tz * w0 * w1 * g.T[2];
+    const TileBox b = tile_at(g, tx, ty, tz);
+    x = b.x0 + r / (b.w1 * b.w2);
+    y = b.y0 + r / b.w2 % b.w1;
+    z = b.z0 + r % b.w2;
 }
 
 __device__ __forceinline__ int nid_of(const Geo& g, int x, int y, int z) {
@@ -245,16 +279,17 @@ __device__ __forceinline__ void tri_weights(float x, float y, float z, float wt[
 
 constexpr int JH = IPIC_JHALO;
 
-// Tile geometry of the particle kernel, from Geo at run time or, for 8x8x8 tiles, as
+// Geometry of a block's tile, from its box at run time or, where all tiles are 8x8x8, as
 // compile-time constants (cell splits and node indices fold into shifts and offsets).
 template <bool FIX8>
 struct TileGeo {
     int T0, T1, T2, TC, nj1, nj2, NJ;
     int nj0;
     float iT2, iT12;
-    __device__ __forceinline__ explicit TileGeo(const Geo& g)
-        : T0(g.T[0]), T1(g.T[1]), T2(g.T[2]), TC(g.TC), nj1(g.nj[1]), nj2(g.nj[2]), NJ(g.NJ), nj0(g.nj[0]),
-          iT2(g.inv_T[2]), iT12(g.inv_T12) {}
+    __device__ __forceinline__ explicit TileGeo(const TileBox& b)
+        : T0(b.w0), T1(b.w1), T2(b.w2), TC(b.cells()), nj1(b.w1 + 1 + 2 * JH), nj2(b.w2 + 1 + 2 * JH),
+          NJ((b.w0 + 1 + 2 * JH) * nj1 * nj2), nj0(b.w0 + 1 + 2 * JH), iT2(__builtin_amdgcn_rcpf((float)b.w2)),
+          iT12(__builtin_amdgcn_rcpf((float)(b.w1 * b.w2))) {}
     // tile-local cell index -> coordinates
     __device__ __forceinline__ void split(int c, int& lx, int& ly, int& lz) const {
         lx = fdivi(c, iT12);
@@ -270,7 +305,7 @@ template <>
 struct TileGeo<true> {
     static constexpr int T0 = 8, T1 = 8, T2 = 8, TC = 512;
     static constexpr int nj0 = 9 + 2 * JH, nj1 = nj0, nj2 = nj0, NJ = nj0 * nj0 * nj0;
-    __device__ __forceinline__ explicit TileGeo(const Geo&) {}
+    __device__ __forceinline__ explicit TileGeo(const TileBox&) {}
     __device__ __forceinline__ void split(int c, int& lx, int& ly, int& lz) const {
         lx = c >> 6;
         ly = (c >> 3) & 7;
@@ -606,7 +641,9 @@ template <int MODE, bool TRACK, int OPT>
 __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     const Geo& g = A.g;
     using TG = TileGeo<(OPT & OPT_FIX8) != 0>;
-    const TG G(g);
+    const int t = A.tile_order ? A.tile_order[blockIdx.x] : (int)blockIdx.x;
+    const TileBox box = tile_box(g, t);
+    const TG G(box);
     constexpr bool SINK = (OPT & OPT_SINK) != 0, REFLECT = (OPT & OPT_REFLECT) != 0;
     constexpr bool DIPOLE = (OPT & OPT_DIPOLE) != 0;  // analytic dipole B, E = 0: no field staging
     extern __shared__ __align__(16) unsigned char smem[];
@@ -630,11 +667,9 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     int* H = (int*)(K0 + K0CAP / 2 * 7);    // WS ints; fewer than K0CAP / 2 leavers wait at a chunk's start
     static_assert(K0CAP / 2 * 7 >= WS, "the run heads fit the leaver buffer's upper half");
 
-    const int t = A.tile_order ? A.tile_order[blockIdx.x] : (int)blockIdx.x;
     const int sl = blockIdx.y;  // this block's slice of the tile's cells
-    const int tx = t / (g.NTl[1] * g.NTl[2]), ty = (t / g.NTl[2]) % g.NTl[1], tz = t % g.NTl[2];
-    const int x0 = tx * G.T0, y0 = ty * G.T1, z0 = tz * G.T2;
-    const int cbase = t * G.TC;
+    const int x0 = box.x0, y0 = box.y0, z0 = box.z0;
+    const int cbase = (OPT & OPT_FIX8) ? t * G.TC : box.first(g);
     const float NaNf = __builtin_nanf("");
     const int fsy = G.T2 + 1, fsx = (G.T1 + 1) * fsy;  // node strides of the LDS field
 
@@ -1223,7 +1258,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     }
     __syncthreads();
     if (MODE != MODE_REBIN) {
-        float* dst = A.jpart + ((long long)t * g.nsl + sl) * 3 * G.NJ;
+        float* dst = A.jpart + ((long long)t * g.nsl + sl) * 3 * g.NJ;
         for (int i = tid; i < 3 * G.NJ; i += NTP) dst[i] = (float)((double)sJ[i] * g.fix_inv);
     }
 }
@@ -1270,14 +1305,15 @@ __device__ __forceinline__ void xyz_of(const Geo& g, int i, int& x, int& y, int&
 // it (every slice of the tile) plus the overflow accumulator (cleared here), rounded once to FP32.
 // The (tile, local node) pairs of axis d whose J partial covers coordinate x, in increasing
 // local index (the order of the jpairs table): without a halo, (x / T, x % T) and, on a tile's
-// low face, (the previous tile, T); with a halo, from the table.
+// low face, (the previous tile, its edge); with a halo, from the table.
 __device__ __forceinline__ int axis_pairs(const FieldArgs& F, int d, int x, int* p) {
     const Geo& g = F.g;
     if (g.jh == 0) {
         const int t = fdivi(x, g.inv_T[d]), l = x - t * g.T[d];
         p[0] = (t << 8) | l;
         if (l != 0) return 1;
-        p[1] = ((t == 0 ? g.NTl[d] - 1 : t - 1) << 8) | g.T[d];
+        const int last = g.NTl[d] - 1;
+        p[1] = t == 0 ? (last << 8) | (g.n[d] - last * g.T[d]) : ((t - 1) << 8) | g.T[d];
         return 2;
     }
     const int* e = F.jpairs + (d * g.nmax + x) * (1 + JPMAX);
@@ -1297,12 +1333,14 @@ __device__ __forceinline__ float4 sum_partials(const FieldArgs& F, int i, int x,
                 const int tb = py[b] >> 8, lb = py[b] & 255;
                 const int tc = pz[cc] >> 8, lc = pz[cc] & 255;
                 const int tile = (ta * g.NTl[1] + tb) * g.NTl[2] + tc;
-                const int l = (la * g.nj[1] + lb) * g.nj[2] + lc;
+                const TileBox bx = tile_at(g, ta, tb, tc);
+                const int h = 1 + 2 * g.jh, nj1 = bx.w1 + h, nj2 = bx.w2 + h, NJ = (bx.w0 + h) * nj1 * nj2;
+                const int l = (la * nj1 + lb) * nj2 + lc;
                 const float* base = F.jpart + (long long)tile * g.nsl * 3 * g.NJ;
                 for (int s = 0; s < F.nsl_read; ++s, base += 3 * g.NJ) {
                     sx += (double)base[l];
-                    sy += (double)base[g.NJ + l];
-                    sz += (double)base[2 * g.NJ + l];
+                    sy += (double)base[NJ + l];
+                    sz += (double)base[2 * NJ + l];
                 }
             }
     // the overflow accumulator, read and cleared only at the nodes that hold deposits
@@ -1656,6 +1694,7 @@ struct ScanSp {
     int* stay;
     int* arr;
     int* tile_total;
+    int* group_total;
 };
 struct ScanArgs {
     Geo g;
@@ -1667,11 +1706,23 @@ __global__ __launch_bounds__(NT) void k_scan_tiles(ScanArgs A) {
     const ScanSp& S = A.sp[blockIdx.y];
     __shared__ int s_w[NT / 64];
     const int t = blockIdx.x;
+    const TileBox b = tile_box(g, t);
+    const int first = b.first(g), cells = b.cells();
     int v = 0;
-    for (int i = threadIdx.x; i < g.TC; i += NT) v += S.cnt_acc[t * g.TC + i];
+    for (int i = threadIdx.x; i < cells; i += NT) v += S.cnt_acc[first + i];
     int tot;
     block_exscan(v, s_w, tot);
     if (threadIdx.x == 0) S.tile_total[t] = tot;
+}
+
+// totals of NT consecutive tiles
+__global__ __launch_bounds__(NT) void k_scan_groups(ScanArgs A) {
+    const ScanSp& S = A.sp[blockIdx.y];
+    __shared__ int s_w[NT / 64];
+    const int t = blockIdx.x * NT + threadIdx.x;
+    int tot;
+    block_exscan(t < A.g.ntiles ? S.tile_total[t] : 0, s_w, tot);
+    if (threadIdx.x == 0) S.group_total[blockIdx.x] = tot;
 }
 
 // Launch order of the particle kernel's tiles for the layout the scans just produced.  A
@@ -1696,6 +1747,7 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
     };
     unsigned long long sum = 0;
     int mx = 0;
+#pragma unroll 8
     for (int t = tid; t < g.ntiles; t += NT) {
         const int v = load(t);
         sum += (unsigned long long)v;
@@ -1723,12 +1775,14 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
         return;
     }
     auto cls = [&](int v) { return 255 - (int)(((long long)v * 255) / mx); };  // heaviest: class 0
+#pragma unroll 8
     for (int t = tid; t < g.ntiles; t += NT) atomicAdd(&s_hist[cls(load(t))], 1);
     __syncthreads();
     int tot;  // exclusive prefix sum of the 256 class counts
     const int first = block_exscan(s_hist[tid], s_w4, tot);
     s_hist[tid] = first;
     __syncthreads();
+#pragma unroll 8
     for (int t = tid; t < g.ntiles; t += NT) order[atomicAdd(&s_hist[cls(load(t))], 1)] = t;
 }
 
@@ -1738,8 +1792,10 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
 // `stay`; the old `stay`, cleared here, the next accumulator).  The cell counters and arrival
 // counters are cleared for the next pass.  Every block adds up the totals of the tiles before its
 // own (16 KB at most from L2 at 128^3): a launch for the bases alone costs more than these reads.
+// With `grouped` (many tiles, where these reads grow with their square) it adds up the totals of groups
+// of NT tiles from k_scan_groups and those of its own group's tiles.
 // A further block orders the tiles for the next push meanwhile.
-__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order) {
+__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order, int grouped) {
     const Geo& g = A.g;
     if ((int)blockIdx.x == g.ntiles) {
         if (blockIdx.y == 0) tile_order_block(A, nsp, order);
@@ -1748,24 +1804,29 @@ __global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* ord
     const ScanSp& S = A.sp[blockIdx.y];
     __shared__ int s_w[NT / 64];
     const int t = blockIdx.x;
-    const int c0 = 2 * threadIdx.x, c1 = c0 + 1;
-    const int id0 = t * g.TC + c0, id1 = t * g.TC + c1;
+    const TileBox b = tile_box(g, t);
+    const int c0 = 2 * threadIdx.x, c1 = c0 + 1, cells = b.cells();
+    const int id0 = b.first(g) + c0, id1 = id0 + 1;
     int v0 = 0, v1 = 0;
-    if (c0 < g.TC) v0 = S.cnt_acc[id0];
-    if (c1 < g.TC) v1 = S.cnt_acc[id1];
-    int before = 0;
+    if (c0 < cells) v0 = S.cnt_acc[id0];
+    if (c1 < cells) v1 = S.cnt_acc[id1];
+    int before = 0, k = threadIdx.x;
+    if (grouped) {  // whole groups, then the tiles of the own group
+        for (; k < t / NT; k += NT) before += S.group_total[k];
+        k = t / NT * NT + threadIdx.x;
+    }
 #pragma unroll 4
-    for (int k = threadIdx.x; k < t; k += NT) before += S.tile_total[k];
+    for (; k < t; k += NT) before += S.tile_total[k];
     int tot, base;
     block_exscan(before, s_w, base);
     const int ex = block_exscan(v0 + v1, s_w, tot) + base;
-    if (c0 < g.TC) {
+    if (c0 < cells) {
         S.seg[id0] = ex;
         S.stay[id0] = 0;
         S.cnt_acc[id0] = 0;
         S.arr[id0] = 0;
     }
-    if (c1 < g.TC) {
+    if (c1 < cells) {
         S.seg[id1] = ex + v0;
         S.stay[id1] = 0;
         S.cnt_acc[id1] = 0;
@@ -1777,6 +1838,9 @@ __global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* ord
 // The same for a grid of few cells, in one launch of one block per species: each wave takes a
 // contiguous share of the cells, adds it up, and scans it 64 cells at a time from the shares before.
 // No tile order: with few tiles every block of the next push is resident at once.
+constexpr int SCAN_GROUPED = 8192;  // tiles above which the scan adds up groups of tiles first:
+                                    // 128^3 (4096 tiles) 37 us so and 32.5 without, 160^3 (8000) both
+                                    // 58, 200^3 (15625) 102 and 111, 256^3 (32768) 260 and 340
 constexpr int SCAN_SMALL = 12288;  // cells up to which this is faster (see launch_scan)
 
 __global__ __launch_bounds__(1024) void k_scan_small(ScanArgs A) {
@@ -2036,11 +2100,8 @@ __global__ __launch_bounds__(256) void k_init(Geo g, const int* start, float* X,
     }
     const int cid = lo;
     const long long idx = p - start[cid];
-    const int t = cid / g.TC, l = cid % g.TC;
-    const int tx = t / (g.NTl[1] * g.NTl[2]), ty = (t / g.NTl[2]) % g.NTl[1], tz = t % g.NTl[2];
-    const int x = tx * g.T[0] + l / (g.T[1] * g.T[2]);
-    const int y = ty * g.T[1] + (l / g.T[2]) % g.T[1];
-    const int z = tz * g.T[2] + l % g.T[2];
+    int x, y, z;
+    cell_of(g, cid, x, y, z);
     const long long row = ((long long)x * g.n[1] + y) * g.n[2] + z;
     uint64_t key = mix64(mix64(mix64(seed) ^ (uint64_t)(uint32_t)species) ^ (uint64_t)row);
     key = mix64(key ^ (uint64_t)idx);
@@ -2282,6 +2343,7 @@ struct Species {
     int* stay_acc = nullptr;
     int* arr = nullptr;
     int* tile_total = nullptr;
+    int* group_total = nullptr;
     int* work = nullptr;  // cells whose arrivals k_canon_large orders (IPIC_FLAG_REPRODUCIBLE)
 };
 
@@ -2376,10 +2438,18 @@ void dfree(ipic_ctx* ctx, void* p) {
     (void)hipFree(p);
 }
 
-int largest_divisor_le(int n, int cap) {
-    for (int t = std::min(n, cap); t >= 1; --t)
+// The tile edge of an axis of n cells: the largest divisor of n from 4 to 8, if it has one, so that all
+// tiles are alike.  Otherwise the fewest tiles of at most 8 cells, the last one shorter, as every
+// tile costs a block and its nodes.  Push of a step, edges from divisors only against these:
+// 47^3 x 32 (edge 1) 1699 -> 85 us, 51x57x33 x 16 (3) 114 -> 55, 27x33x39 x 32 (3) 60 -> 48, 62^3 (2),
+// uneven, 769 -> 625.  For an edge of 4 it is about even: 44x52x44 x 24 82 -> 73 but the
+// field phase 19 -> 29 (tiles of 8 are few enough there to be split), and an uneven 44^3 114 -> 213 (its
+// heaviest tile).
+int tile_edge(int n) {
+    for (int t = std::min(n, 8); t >= 4; --t)
         if (n % t == 0) return t;
-    return 1;
+    const int tiles = (n + 7) / 8;
+    return (n + tiles - 1) / tiles;
 }
 
 // per axis, the (tile, local node) pairs whose J partial region [tile*T - 1, tile*T + T + 2)
@@ -2392,9 +2462,10 @@ int build_jpairs(const Geo& g, std::vector<int>& tab) {
             for (int l = 0; l < g.nj[d]; ++l) {
                 int s = (x + g.jh - l) % g.n[d];
                 if (s < 0) s += g.n[d];
-                if (s % g.T[d] == 0) {
+                const int t = s / g.T[d], w = std::min(g.T[d], g.n[d] - s);
+                if (s % g.T[d] == 0 && l < w + 1 + 2 * g.jh) {
                     if (e[0] >= JPMAX) return -1;
-                    e[1 + e[0]] = ((s / g.T[d]) << 8) | l;
+                    e[1 + e[0]] = (t << 8) | l;
                     e[0]++;
                 }
             }
@@ -2467,7 +2538,7 @@ ScanArgs scan_args(ipic_ctx* ctx) {
     A.g = ctx->g;
     for (int s = 0; s < ctx->d.nspecies; ++s) {
         Species& S = ctx->sp[s];
-        A.sp[s] = ScanSp{S.cnt_acc, S.stay_acc, S.seg, S.start, S.stay, S.arr, S.tile_total};
+        A.sp[s] = ScanSp{S.cnt_acc, S.stay_acc, S.seg, S.start, S.stay, S.arr, S.tile_total, S.group_total};
     }
     return A;
 }
@@ -2510,7 +2581,9 @@ int launch_particles(ipic_ctx* ctx, int mode) {
     const bool dip = (ctx->d.flags & IPIC_FLAG_DIPOLE_MOVER) != 0;
     const size_t lds =
         (size_t)particle_layout(g.NJ, g.TC, (mode == MODE_PUSH && !dip) ? field_nodes(g) : 0, ctx->track).total;
-    const int opt = ((g.T[0] == 8 && g.T[1] == 8 && g.T[2] == 8) ? OPT_FIX8 : 0) | (g.sink ? OPT_SINK : 0) |
+    bool fix8 = true;
+    for (int k = 0; k < 3; ++k) fix8 = fix8 && g.T[k] == 8 && g.n[k] % 8 == 0;
+    const int opt = (fix8 ? OPT_FIX8 : 0) | (g.sink ? OPT_SINK : 0) |
                     (g.reflect ? OPT_REFLECT : 0) | (dip ? OPT_DIPOLE : 0);
     hipStream_t st = ctx->stream;
     if (ctx->track) {
@@ -2540,7 +2613,11 @@ int launch_scan(ipic_ctx* ctx) {
         hipLaunchKernelGGL(k_scan_small, dim3(ns), dim3(1024), 0, ctx->stream, A);
     } else {
         hipLaunchKernelGGL(k_scan_tiles, dim3(ctx->g.ntiles, ns), dim3(NT), 0, ctx->stream, A);
-        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order);
+        const int grouped = ctx->g.ntiles > SCAN_GROUPED;
+        if (grouped)
+            hipLaunchKernelGGL(k_scan_groups, dim3((ctx->g.ntiles + NT - 1) / NT, ns), dim3(NT), 0, ctx->stream, A);
+        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order,
+                           grouped);
     }
     HIPCK(ctx, hipGetLastError());
     for (int s = 0; s < ns; ++s) {  // the roles k_scan_cells gave the arrays
@@ -2853,19 +2930,9 @@ int read_slots(ipic_ctx* ctx, int s, long long* slots) {
     return 0;
 }
 
-// cell coordinates of a tile-major cell id
-inline void cid_xyz(const Geo& g, int cid, int& x, int& y, int& z) {
-    const int t = cid / g.TC, l = cid % g.TC;
-    const int tx = t / (g.NTl[1] * g.NTl[2]), ty = (t / g.NTl[2]) % g.NTl[1], tz = t % g.NTl[2];
-    x = tx * g.T[0] + l / (g.T[1] * g.T[2]);
-    y = ty * g.T[1] + (l / g.T[2]) % g.T[1];
-    z = tz * g.T[2] + l % g.T[2];
-}
-
 inline int host_cid(const Geo& g, int x, int y, int z) {
-    const int tx = x / g.T[0], ty = y / g.T[1], tz = z / g.T[2];
-    const int lx = x - tx * g.T[0], ly = y - ty * g.T[1], lz = z - tz * g.T[2];
-    return ((tx * g.NTl[1] + ty) * g.NTl[2] + tz) * g.TC + (lx * g.T[1] + ly) * g.T[2] + lz;
+    const TileBox b = tile_at(g, x / g.T[0], y / g.T[1], z / g.T[2]);
+    return b.first(g) + ((x - b.x0) * b.w1 + (y - b.y0)) * b.w2 + z - b.z0;
 }
 
 int alloc_species_buffers(ipic_ctx* ctx, int s, long long cap) {
@@ -3072,13 +3139,13 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         Geo& g = ctx->g;
         for (int k = 0; k < 3; ++k) {
             g.n[k] = d.n[k];
-            int T = d.tile[k] > 0 ? d.tile[k] : largest_divisor_le(d.n[k], 8);
-            if (T > 8 || d.n[k] % T != 0) {
+            const int T = d.tile[k] > 0 ? d.tile[k] : tile_edge(d.n[k]);
+            if (T > 8 || (d.tile[k] > 0 && d.n[k] % T != 0)) {
                 delete ctx;
                 return fail(nullptr, IPIC_E_ARG, "tile size must divide the grid and be at most 8");
             }
             g.T[k] = T;
-            g.NTl[k] = d.n[k] / T;
+            g.NTl[k] = (d.n[k] + T - 1) / T;
             g.jh = IPIC_JHALO;
             g.nj[k] = T + 1 + 2 * g.jh;
             g.w[k] = (float)d.cell_width[k];
@@ -3107,7 +3174,6 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         g.inv_vol = (float)(1.0 / (d.cell_width[0] * d.cell_width[1] * d.cell_width[2]));
         g.pi_c = (float)(M_PI * d.c);
         for (int k = 0; k < 3; ++k) g.inv_T[k] = 1.0f / (float)g.T[k];
-        g.inv_T12 = 1.0f / (float)(g.T[1] * g.T[2]);
         {
             // fixed-point scale of the LDS J accumulator: one particle at speed c contributes about
             // 2^30 units, leaving 2^33 of headroom for the sums of a tile node
@@ -3172,6 +3238,7 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             rc = rc ? rc : dalloc(ctx, &S.stay_acc, nc);
             rc = rc ? rc : dalloc(ctx, &S.arr, nc);
             rc = rc ? rc : dalloc(ctx, &S.tile_total, (size_t)g.ntiles);
+            rc = rc ? rc : dalloc(ctx, &S.group_total, ((size_t)g.ntiles + NT - 1) / NT);
             if (d.flags & IPIC_FLAG_REPRODUCIBLE) rc = rc ? rc : dalloc(ctx, &S.work, nc + 1);
         }
         if (!rc) {
@@ -3342,7 +3409,7 @@ int ipic_gpu_init_particles(ipic_ctx* ctx, int32_t species, const int32_t* ppc, 
         long long total = 0;
         for (int cid = 0; cid < nc; ++cid) {
             int x, y, z;
-            cid_xyz(g, cid, x, y, z);
+            cell_of(g, cid, x, y, z);
             const int row = (x * g.n[1] + y) * g.n[2] + z;
             const long long k = ppc ? ppc[row] : uniform_ppc;
             if (k < 0) return fail(ctx, IPIC_E_ARG, "negative particles per cell");
@@ -3546,8 +3613,8 @@ int ipic_gpu_field_step(ipic_ctx* ctx, int32_t use_operator, ipic_step_stats* st
         if (use_operator && !ctx->op_on) return fail(ctx, IPIC_E_STATE, "no field operator set");
         ipic_step_stats st{};
         if (int rc = field_phase(ctx, use_operator != 0, &st)) return rc;
-        // (the runtime's wait: a phase is many short kernels that the host queues ahead of, and one
-        // more at their end costs 3 of 98 us at 64^3 with 8 substeps)
+        // (the runtime's wait: a phase is a few short kernels that the host queues ahead of, and one
+        // more at their end costs 3 us)
         HIPCK(ctx, hipStreamSynchronize(ctx->stream));
         if (stats) {
             stats->ms_field += st.ms_field;
@@ -3686,7 +3753,7 @@ int ipic_gpu_cell_counts(ipic_ctx* ctx, int32_t species, int64_t* counts) {
             HIPCK(ctx, hipMemcpy(st.data(), ctx->sp[s].start, (nc + 1) * sizeof(int), hipMemcpyDeviceToHost));
             for (int cid = 0; cid < nc; ++cid) {
                 int x, y, z;
-                cid_xyz(g, cid, x, y, z);
+                cell_of(g, cid, x, y, z);
                 counts[(x * g.n[1] + y) * g.n[2] + z] += st[cid + 1] - st[cid];
             }
         }

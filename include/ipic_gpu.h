@@ -77,7 +77,8 @@ typedef struct ipic_desc {
                                      (cell.h:1123-1128, planetRadius / objectCenter) */
     double sink_center[3];
     double sink_radius;
-    int32_t tile[3];              /* cells per tile along each axis; 0 = automatic (<= 8, divides n) */
+    int32_t tile[3];              /* cells per tile along each axis; 0 = automatic: at most 8, and the
+                                     last tile of an axis may be shorter; given ones divide n */
     uint32_t flags;               /* IPIC_FLAG_* */
     double dipole_moment;         /* -externalMagneticField.z * planetRadius^3 (cell.h:921), read
                                      with IPIC_FLAG_DIPOLE_MOVER */
