@@ -126,7 +126,7 @@ struct PushArgs {
     unsigned char* jmark; // jmark[i] = 1: node i holds overflow deposits
     unsigned long long* removed;
     int* err;             // set to nonzero when a consistency guard fires
-    const int* tile_order;  // block -> tile (a permutation), or null for tile = block
+    const int2* order;    // block -> tile and slice (tile_order_block), or null for the plain order
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -641,7 +641,15 @@ template <int MODE, bool TRACK, int OPT>
 __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     const Geo& g = A.g;
     using TG = TileGeo<(OPT & OPT_FIX8) != 0>;
-    const int t = A.tile_order ? A.tile_order[blockIdx.x] : (int)blockIdx.x;
+    // this block's tile t, and its cells: slice sl of nsl
+    int t = blockIdx.x % (unsigned)g.ntiles, sl = blockIdx.x / (unsigned)g.ntiles, nsl = g.nsl;
+    if (A.order) {
+        const int2 o = A.order[blockIdx.x];
+        if (o.x < 0) return;  // no more slices
+        t = o.x;
+        sl = o.y & 0xffff;
+        nsl = o.y >> 16;
+    }
     const TileBox box = tile_box(g, t);
     const TG G(box);
     constexpr bool SINK = (OPT & OPT_SINK) != 0, REFLECT = (OPT & OPT_REFLECT) != 0;
@@ -667,7 +675,6 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
     int* H = (int*)(K0 + K0CAP / 2 * 7);    // WS ints; fewer than K0CAP / 2 leavers wait at a chunk's start
     static_assert(K0CAP / 2 * 7 >= WS, "the run heads fit the leaver buffer's upper half");
 
-    const int sl = blockIdx.y;  // this block's slice of the tile's cells
     const int x0 = box.x0, y0 = box.y0, z0 = box.z0;
     const int cbase = (OPT & OPT_FIX8) ? t * G.TC : box.first(g);
     const float NaNf = __builtin_nanf("");
@@ -775,7 +782,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         for (int q = 0; q < ns; ++q)
             for (int i = tid; i <= G.TC; i += NTP) s_segs[q * (G.TC + 1) + i] = A.sp[sg + q].seg[cbase + i];
         __syncthreads();
-        // the block's cells [clo, chi): slice sl of g.nsl at equal particle counts; cells of
+        // the block's cells [clo, chi): slice sl of nsl at equal particle counts; cells of
         // wave w: [s_wlo[w], s_wlo[w+1]), the slice split again at equal particle counts.  Each
         // cut goes to the cell boundary nearest to it: at the next one instead, a wave of a slice of
         // four cells of about equal size often got two of them (8^3 cells, 512 per cell: 81 against
@@ -792,8 +799,8 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                 return lo > 0 && target - s_seg[lo - 1] < s_seg[lo] - target ? lo - 1 : lo;
             };
             const long long tot = (long long)s_seg[G.TC] - s_seg[0];
-            const int clo = (sl == 0) ? 0 : nearest(s_seg[0] + tot * sl / g.nsl);
-            const int chi = (sl == g.nsl - 1) ? G.TC : nearest(s_seg[0] + tot * (sl + 1) / g.nsl);
+            const int clo = (sl == 0) ? 0 : nearest(s_seg[0] + tot * sl / nsl);
+            const int chi = (sl == nsl - 1) ? G.TC : nearest(s_seg[0] + tot * (sl + 1) / nsl);
             const long long sub = (long long)s_seg[chi] - s_seg[clo];
             s_wlos[tid] = (w == 0) ? clo
                         : (w == NW ? chi : max(clo, min(chi, nearest(s_seg[clo] + sub * w / NW))));
@@ -1271,9 +1278,21 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
         }
     }
     __syncthreads();
-    if (MODE != MODE_REBIN) {
+    if (MODE != MODE_REBIN && sl < g.nsl) {
         float* dst = A.jpart + ((long long)t * g.nsl + sl) * 3 * g.NJ;
         for (int i = tid; i < 3 * G.NJ; i += NTP) dst[i] = (float)((double)sJ[i] * g.fix_inv);
+    } else if (MODE != MODE_REBIN) {  // a slice beyond those with partials of their own: the global accumulator
+        for (int l = tid; l < G.NJ; l += NTP) {
+            const long long jx = sJ[l], jy = sJ[G.NJ + l], jz = sJ[2 * G.NJ + l];
+            if ((jx | jy | jz) == 0) continue;
+            const int a = l / (G.nj1 * G.nj2), r = l - a * G.nj1 * G.nj2, b = r / G.nj2, c = r - b * G.nj2;
+            const int gid = nid_of(g, wrapc(x0 + a - JH, g.n[0]), wrapc(y0 + b - JH, g.n[1]), wrapc(z0 + c - JH, g.n[2]));
+            long long* o = A.jover + 3 * (long long)gid;
+            __hip_atomic_store(&A.jmark[gid], (unsigned char)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 0, jx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 1, jy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(o + 2, jz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
@@ -1739,25 +1758,51 @@ __global__ __launch_bounds__(NT) void k_scan_groups(ScanArgs A) {
     if (threadIdx.x == 0) S.group_total[blockIdx.x] = tot;
 }
 
-// Launch order of the particle kernel's tiles for the layout the scans just produced.  A
-// block's time grows with its tile's particles.  With an uneven load (the heaviest tile more
-// than 25 % above the mean) the heaviest tiles go first (longest-processing-time order over 256
-// load classes), so that the blocks that start last are light.  Otherwise tile b goes to block b:
-// neighbouring tiles run at the same time on different XCDs (blocks are dealt round-robin over the
+// Launch order of the particle kernel's blocks for the layout the scans just produced: (tile, slice and
+// the tile's number of slices), with (-1, 0) for the blocks left over.  A block's time grows with
+// its particles.  With an uneven load (the heaviest tile more than 25 % above the mean) a tile gets one
+// slice for every 1 / extra of all particles that it holds, at least the nsl that have partials of
+// their own, and the heaviest slices go first (longest-processing-time order over 256 load classes),
+// so that the blocks that start last are light.  With `extra` two blocks per CU the push of an uneven
+// 96^3 (300 particles a cell at the densest, 30 outside) takes 655 us instead of 992, whose end
+// was its heaviest tile alone; 62^3 145 (512), 47^3 84 (200), 53^3 64 (186); with one per CU 992, 214,
+// 134, 87; with four 650, 156, 106, 85; all tiles in three slices 722 at 96^3 and 60 more for the E pass.
+// Otherwise tile b goes to block b: neighbouring tiles run at the same time on different XCDs (blocks are dealt round-robin over the
 // 8 XCDs).  Scrambled over the grid the push took 1.3 % more at 128^3 x 32 and 4 % more at
-// 96^3 x 32, an eighth of the grid for each XCD in turn 2 % more.  Any permutation gives the same
-// results: the order only schedules.
-__device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
+// 96^3 x 32, an eighth of the grid for each XCD in turn 2 % more.  Any order and any number of slices
+// give the same particles, and J up to the rounding of its partials.
+__device__ void tile_order_block(const ScanArgs& A, int nsp, int2* order, int extra) {
     const Geo& g = A.g;
     __shared__ unsigned long long s_sum[NT / 64];
     __shared__ int s_max[NT / 64], s_w4[NT / 64];
     __shared__ int s_hist[256];
     static_assert(NT == 256, "one thread per load class");
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int blocks = g.ntiles * g.nsl + extra;
     auto load = [&](int t) {
         int v = 0;
         for (int sp = 0; sp < nsp; ++sp) v += A.sp[sp].tile_total[t];
         return v;
+    };
+    // over the block: the sum of a, the maximum of m
+    auto reduce = [&](unsigned long long& a, int& m) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            a += __shfl_xor(a, d, 64);
+            m = max(m, __shfl_xor(m, d, 64));
+        }
+        __syncthreads();
+        if (lane == 0) {
+            s_sum[wid] = a;
+            s_max[wid] = m;
+        }
+        __syncthreads();
+        a = 0;
+        m = 0;
+        for (int w = 0; w < NT / 64; ++w) {
+            a += s_sum[w];
+            m = max(m, s_max[w]);
+        }
     };
     unsigned long long sum = 0;
     int mx = 0;
@@ -1767,37 +1812,45 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
         sum += (unsigned long long)v;
         mx = max(mx, v);
     }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        sum += __shfl_xor(sum, d, 64);
-        mx = max(mx, __shfl_xor(mx, d, 64));
-    }
-    if (lane == 0) {
-        s_sum[wid] = sum;
-        s_max[wid] = mx;
-    }
-    s_hist[tid] = 0;
-    __syncthreads();
-    sum = 0;
-    mx = 0;
-    for (int w = 0; w < NT / 64; ++w) {
-        sum += s_sum[w];
-        mx = max(mx, s_max[w]);
-    }
+    reduce(sum, mx);
     if ((double)mx * g.ntiles <= 1.25 * (double)sum || mx == 0) {
-        for (int b = tid; b < g.ntiles; b += NT) order[b] = b;
+        for (int b = tid; b < blocks; b += NT) {
+            const int sl = b / g.ntiles;
+            order[b] = sl < g.nsl ? make_int2(b - sl * g.ntiles, sl | g.nsl << 16) : make_int2(-1, 0);
+        }
         return;
     }
-    auto cls = [&](int v) { return 255 - (int)(((long long)v * 255) / mx); };  // heaviest: class 0
+    // v particles make ceil(v / part) slices, at most v / part beyond the first, and sum / part < extra
+    const unsigned part = (unsigned)(sum / (unsigned)extra) + 1u;
+    const int most = max(g.nsl, g.TC / 4);
+    auto slices = [&](int v) { return min(max((int)(((unsigned)v + part - 1u) / part), g.nsl), most); };
+    unsigned long long none = 0;
+    int heavy = 0;  // the heaviest slice
 #pragma unroll 8
-    for (int t = tid; t < g.ntiles; t += NT) atomicAdd(&s_hist[cls(load(t))], 1);
+    for (int t = tid; t < g.ntiles; t += NT) {
+        const int v = load(t);
+        heavy = max(heavy, v / slices(v));
+    }
+    s_hist[tid] = 0;
+    reduce(none, heavy);
+    heavy = max(heavy, 1);
+    // heaviest: class 0
+    auto cls = [&](int v, int m) { return 255 - (int)(((long long)(v / m) * 255) / heavy); };
+#pragma unroll 8
+    for (int t = tid; t < g.ntiles; t += NT) {
+        const int v = load(t), m = slices(v);
+        atomicAdd(&s_hist[cls(v, m)], m);
+    }
     __syncthreads();
     int tot;  // exclusive prefix sum of the 256 class counts
     const int first = block_exscan(s_hist[tid], s_w4, tot);
     s_hist[tid] = first;
     __syncthreads();
-#pragma unroll 8
-    for (int t = tid; t < g.ntiles; t += NT) order[atomicAdd(&s_hist[cls(load(t))], 1)] = t;
+    for (int t = tid; t < g.ntiles; t += NT) {
+        const int v = load(t), m = slices(v), p = atomicAdd(&s_hist[cls(v, m)], m);
+        for (int k = 0; k < m; ++k) order[p + k] = make_int2(t, k | m << 16);
+    }
+    for (int b = tot + tid; b < blocks; b += NT) order[b] = make_int2(-1, 0);
 }
 
 // New starts = tile base + in-tile exclusive prefix of the counts, written over the old
@@ -1808,16 +1861,16 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int* order) {
 // own (16 KB at most from L2 at 128^3): a launch for the bases alone costs more than these reads.
 // With `grouped` (many tiles, where these reads grow with their square) it adds up the totals of groups
 // of NT tiles from k_scan_groups and those of its own group's tiles.
-// A further block orders the tiles for the next push meanwhile.
-__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int* order, int grouped) {
+// The first block orders the blocks of the next push meanwhile.
+__global__ __launch_bounds__(NT) void k_scan_cells(ScanArgs A, int nsp, int2* order, int extra, int grouped) {
     const Geo& g = A.g;
-    if ((int)blockIdx.x == g.ntiles) {
-        if (blockIdx.y == 0) tile_order_block(A, nsp, order);
+    if (blockIdx.x == 0) {
+        if (blockIdx.y == 0) tile_order_block(A, nsp, order, extra);
         return;
     }
     const ScanSp& S = A.sp[blockIdx.y];
     __shared__ int s_w[NT / 64];
-    const int t = blockIdx.x;
+    const int t = blockIdx.x - 1;
     const TileBox b = tile_box(g, t);
     const int c0 = 2 * threadIdx.x, c1 = c0 + 1, cells = b.cells();
     const int id0 = b.first(g) + c0, id1 = id0 + 1;
@@ -2386,8 +2439,9 @@ struct ipic_ctx {
     int* jpairs = nullptr;
     unsigned long long* removed = nullptr;
     int* derr = nullptr;
-    int* tile_order = nullptr;     // launch order of the particle kernel's tiles
-    bool order_valid = false;      // tile_order describes the current layout's loads
+    int2* order = nullptr;         // launch order of the particle kernel's blocks
+    int extra = 512;               // blocks it may take for the slices of heavy tiles, two per CU
+    bool order_valid = false;      // `order` describes the current layout's loads
     double* red = nullptr;
     int red_blocks = 1024;
     Species sp[IPIC_MAX_SPECIES];
@@ -2452,15 +2506,15 @@ void dfree(ipic_ctx* ctx, void* p) {
     (void)hipFree(p);
 }
 
-// The tile edge of an axis of n cells: the largest divisor of n from 4 to 8, if it has one, so that all
-// tiles are alike.  Otherwise the fewest tiles of at most 8 cells, the last one shorter, as every
-// tile costs a block and its nodes.  Push of a step, edges from divisors only against these:
-// 47^3 x 32 (edge 1) 1699 -> 85 us, 51x57x33 x 16 (3) 114 -> 55, 27x33x39 x 32 (3) 60 -> 48, 62^3 (2),
-// uneven, 769 -> 625.  For an edge of 4 it is about even: 44x52x44 x 24 82 -> 73 but the
-// field phase 19 -> 29 (tiles of 8 are few enough there to be split), and an uneven 44^3 114 -> 213 (its
-// heaviest tile).
-int tile_edge(int n) {
-    for (int t = std::min(n, 8); t >= 4; --t)
+// The tile edge of an axis of n cells: the fewest tiles of at most 8 cells, the last one shorter.  Every
+// tile costs a block and its nodes.  Push of a step against edges that divide n (the largest up to
+// 8): 47^3 x 32 (edge 1) 85 us and 1699, 51x57x33 x 16 (3) 55 and 114, 27x33x39 x 32 (3) 48 and 60,
+// 44x52x44 x 24 (4) 69 and 83, 65^3 x 24 (5) 133 and 161, 100^3 x 8 (5) 203 and 292, 60^3 x 24 (6) 127
+// and 136.  On a grid of few tiles, where tiles of 8 would be split into slices and their
+// partials summed, an edge of 5 to 8 that divides n is kept (the largest; 45^3 x 24: push and field phase
+// 80 us with 5, 101 with 8; an edge of 4, 44x52x44 x 24, 102 and 98).
+int tile_edge(int n, bool few) {
+    for (int t = std::min(n, 8); few && t >= 5; --t)
         if (n % t == 0) return t;
     const int tiles = (n + 7) / 8;
     return (n + tiles - 1) / tiles;
@@ -2517,7 +2571,7 @@ PushArgs push_args(ipic_ctx* ctx) {
     A.jmark = ctx->jmark;
     A.removed = ctx->removed;
     A.err = ctx->derr;
-    A.tile_order = ctx->order_valid ? ctx->tile_order : nullptr;
+    A.order = ctx->order_valid ? ctx->order : nullptr;
     return A;
 }
 
@@ -2591,7 +2645,7 @@ int launch_particles(ipic_ctx* ctx, int mode) {
     }
     PushArgs A = push_args(ctx);
     const Geo& g = ctx->g;
-    dim3 grid(g.ntiles, g.nsl), block(NTP);
+    dim3 grid(g.ntiles * g.nsl + (A.order ? ctx->extra : 0)), block(NTP);
     const bool dip = (ctx->d.flags & IPIC_FLAG_DIPOLE_MOVER) != 0;
     const size_t lds =
         (size_t)particle_layout(g.NJ, g.TC, (mode == MODE_PUSH && !dip) ? field_nodes(g) : 0, ctx->track).total;
@@ -2630,8 +2684,8 @@ int launch_scan(ipic_ctx* ctx) {
         const int grouped = ctx->g.ntiles > SCAN_GROUPED;
         if (grouped)
             hipLaunchKernelGGL(k_scan_groups, dim3((ctx->g.ntiles + NT - 1) / NT, ns), dim3(NT), 0, ctx->stream, A);
-        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->tile_order,
-                           grouped);
+        hipLaunchKernelGGL(k_scan_cells, dim3(ctx->g.ntiles + 1, ns), dim3(NT), 0, ctx->stream, A, ns, ctx->order,
+                           ctx->extra, grouped);
     }
     HIPCK(ctx, hipGetLastError());
     for (int s = 0; s < ns; ++s) {  // the roles k_scan_cells gave the arrays
@@ -3151,9 +3205,18 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         }
         ctx->track = (d.flags & IPIC_FLAG_TRACK_IDS) != 0;
         Geo& g = ctx->g;
+        int cus = 256, dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+            cus = 256;
+        long long tiles = 1;
+        for (int k = 0; k < 3; ++k) {
+            const int T = d.tile[k] > 0 ? d.tile[k] : tile_edge(d.n[k], false);
+            tiles *= (d.n[k] + T - 1) / T;
+        }
         for (int k = 0; k < 3; ++k) {
             g.n[k] = d.n[k];
-            const int T = d.tile[k] > 0 ? d.tile[k] : tile_edge(d.n[k]);
+            const int T = d.tile[k] > 0 ? d.tile[k] : tile_edge(d.n[k], tiles < 2 * cus);
             if (T > 8 || (d.tile[k] > 0 && d.n[k] % T != 0)) {
                 delete ctx;
                 return fail(nullptr, IPIC_E_ARG, "tile size must divide the grid and be at most 8");
@@ -3173,12 +3236,9 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             // One block per tile leaves most CUs idle on a grid of few tiles (8^3 cells: one tile).
             // The particle kernel then splits each tile's cells among several blocks, up to two
             // blocks per CU and at least as many cells per block as it has waves.
-            int cus = 256, dev = 0;
-            if (hipGetDevice(&dev) != hipSuccess ||
-                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-                cus = 256;
             const int want = (2 * cus + g.ntiles - 1) / g.ntiles;
             g.nsl = std::max(1, std::min(want, g.TC / NW));
+            ctx->extra = 2 * cus;
         }
         g.ncell = (int)ncell;
         g.NJ = g.nj[0] * g.nj[1] * g.nj[2];
@@ -3239,7 +3299,7 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         rc = rc ? rc : dalloc(ctx, &ctx->jpairs, jp.size());
         rc = rc ? rc : dalloc(ctx, &ctx->removed, 1);
         rc = rc ? rc : dalloc(ctx, &ctx->derr, 1);
-        rc = rc ? rc : dalloc(ctx, &ctx->tile_order, (size_t)g.ntiles);
+        rc = rc ? rc : dalloc(ctx, &ctx->order, (size_t)g.ntiles * g.nsl + ctx->extra);
         rc = rc ? rc : dalloc(ctx, &ctx->red, (size_t)ctx->red_blocks * 5);
         for (int s = 0; s < d.nspecies && !rc; ++s) {
             Species& S = ctx->sp[s];
