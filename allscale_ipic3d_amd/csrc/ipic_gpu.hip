@@ -1370,6 +1370,7 @@ __device__ __forceinline__ float4 sum_partials(const FieldArgs& F, int i, int x,
                 const int h = 1 + 2 * g.jh, nj1 = bx.w1 + h, nj2 = bx.w2 + h, NJ = (bx.w0 + h) * nj1 * nj2;
                 const int l = (la * nj1 + lb) * nj2 + lc;
                 const float* base = F.jpart + (long long)tile * g.nsl * 3 * g.NJ;
+#pragma unroll 4
                 for (int s = 0; s < F.nsl_read; ++s, base += 3 * g.NJ) {
                     sx += (double)base[l];
                     sy += (double)base[NJ + l];
@@ -2718,16 +2719,18 @@ int launch_canon(ipic_ctx* ctx) {
 
 int launch_jsum(ipic_ctx* ctx);
 
-// Reduces the block slices of the partials (a no-op with one slice per tile); F reads one slice
-// afterwards.
+// Reduces the block slices of the partials; F reads one slice afterwards.  A few slices are left to
+// the node sums, whose reads of them are in flight together: less than a launch (field phase of 47^3, 3
+// slices, 27.6 -> 23 us, 45x28x31, 4, 27.4 -> 24.4, 40^3, 5, 24 -> 22, 32^3, 8, even).
+constexpr int SLICES_READ = 6;
 int slice_sum(ipic_ctx* ctx, FieldArgs& F) {
     const Geo& g = ctx->g;
-    if (g.nsl > 1) {
+    if (g.nsl > SLICES_READ) {
         hipLaunchKernelGGL(k_slice_sum, dim3(g.ntiles * ((3 * g.NJ + 31) / 32)), dim3(256), 0, ctx->stream, g,
                            ctx->jpart);
         HIPCK(ctx, hipGetLastError());
+        F.nsl_read = 1;
     }
-    F.nsl_read = 1;
     return 0;
 }
 
