@@ -122,6 +122,8 @@ __device__ __forceinline__ v4f mma(v4s a, v4s b, v4f c) { return __builtin_amdgc
 template <int CIN, int COUT, int BY>
 __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
     constexpr int HY = BY + 2, HV = HX * HY * HZ;
+    constexpr bool WHOLE = 4 % BY == 0;  // n[1] is a multiple of 4; else its last bricks may be shorter
+    constexpr bool AHEAD = BY <= 4;      // the next brick's halo in registers while this one computes
     constexpr bool K32 = CIN == 32 && COUT == 32;
     typedef typename Frag<K32>::T F;
     constexpr int RB = CIN * 2;             // LDS bytes per halo voxel and per weight row
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
     __shared__ __align__(16) unsigned char sw[27 * COUT * RB];  // the layer's weights, all bricks
     __shared__ __align__(16) unsigned char sx[2][HV * RB];      // the two current bricks' halos
     const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
-    const int nbz = n2 / BZ, nby = n1 / BY;
+    const int nbz = n2 / BZ, nby = (n1 + BY - 1) / BY;
     // the block's two halves (4 waves each) work on bricks 2 p and 2 p + 1 of pair p
     const int half = threadIdx.x >> 8, ht = threadIdx.x & 255;
     const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) & 3;
@@ -211,16 +213,18 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
                 *(v4u*)(hx_ + ((j * RPI + fq) * HZ + fz) * RB + ((fp ^ swz(fz)) * 16)) = pre[j];
         }
         __syncthreads();
-        if (pr + 1 < p_hi && bb + 2 < nbricks) fetch(bb + 2);
+        if (AHEAD && pr + 1 < p_hi && bb + 2 < nbricks) fetch(bb + 2);
         if (!mine) continue;
         const int bz = bb % nbz, by = (bb / nbz) % nby, bx = bb / (nbz * nby);
         // this lane's results of row y: NT values of 4 channels, at offset o + y n2 COUT, the
         // second 8 voxels further
         const long long o = ((((long long)bx * BX + w) * n1 + by * BY) * n2 + bz * BZ + (hi ? m - 8 : m)) * COUT + c0;
+        const int rows = WHOLE ? BY : min(BY, n1 - by * BY);
         v4f res[BY][NT];
         if (a.res)
 #pragma unroll
             for (int y = 0; y < BY; ++y)
+                if (y < rows)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) res[y][t] = *(const v4f*)(a.res + o + ((long long)y * n2 + 8 * t) * COUT);
 
@@ -267,6 +271,7 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
         // (a row's halves from two instructions reach memory as partial lines).
 #pragma unroll
         for (int y = 0; y < BY; ++y) {
+            if (y >= rows) break;
             v4f v[NT];
             if constexpr (NT == 2) {
 #pragma unroll
@@ -299,6 +304,7 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
                 }
             }
         }
+        if (!AHEAD && pr + 1 < p_hi && bb + 2 < nbricks) fetch(bb + 2);
     }
 }
 
@@ -755,18 +761,24 @@ int conv(const int32_t n[3], const uint16_t* x, const uint16_t* w, const float* 
          const float* res, float* outf, uint16_t* outb, int act, hipStream_t st) {
     ConvArgs a{{n[0], n[1], n[2]}, x, w, bias, zs, res, outf, outb, act};
     // One persistent block per CU: the weights are staged in LDS once per block, and its two
-    // halves work on two bricks at a time.  Bricks of 4 or of 2 rows: a round of bricks costs about
-    // its rows and two rows' time for the halo and the latency, so the shorter ones pay where
-    // the taller ones leave halves idle (32^3, 128 tall bricks for 512 halves: 7.7 against 9.0 us,
-    // first conv of a block) and not in whole rounds (64^3: 23.9 against 19.2 us) or nearly so
-    // (36 x 60 x 64, 540 tall bricks: 17.8 against 16.8 us).
+    // halves work on two bricks at a time.  A round of bricks costs about its rows and two rows' time
+    // for the halo and the latency: of bricks of 1 to 5 rows (the last of a column shorter where the
+    // rows do not divide n[1]) those with the least of it are taken.  The whole network with 1, 2, 3, 4
+    // and 5 rows: 32^3 89, 99, 109, 117, 134 us; 52x56x32 171, 161, 131, 136, 154; 64^3 365, 299,
+    // 288, 259, 290; 36x60x64 (540 bricks of 4 rows for 512 halves) 245, 217, 195, 217, 175.
     const int planes = (n[0] / BX) * (n[2] / BZ), halves = 2 * cu_count();
-    auto rounds = [&](int rows) { return (planes * (n[1] / rows) + halves - 1) / halves; };
+    auto bricks = [&](int rows) { return planes * ((n[1] + rows - 1) / rows); };
+    auto cost = [&](int rows) { return (bricks(rows) + halves - 1) / halves * (rows + 2); };
     auto go = [&](auto kernel, int rows) {
-        const int bricks = planes * (n[1] / rows), pairs = (bricks + 1) / 2;
-        hipLaunchKernelGGL(kernel, dim3(std::min(pairs, cu_count())), dim3(512), 0, st, a, bricks);
+        hipLaunchKernelGGL(kernel, dim3(std::min((bricks(rows) + 1) / 2, cu_count())), dim3(512), 0, st, a, bricks(rows));
     };
-    if (2 * rounds(2) < 3 * rounds(4)) go(k_conv<CIN, COUT, 2>, 2);
+    int rows = 4;
+    for (int r : {5, 3, 2, 1})
+        if (cost(r) < cost(rows)) rows = r;
+    if (rows == 1) go(k_conv<CIN, COUT, 1>, 1);
+    else if (rows == 2) go(k_conv<CIN, COUT, 2>, 2);
+    else if (rows == 3) go(k_conv<CIN, COUT, 3>, 3);
+    else if (rows == 5) go(k_conv<CIN, COUT, 5>, 5);
     else go(k_conv<CIN, COUT, 4>, 4);
     NOPCK(hipGetLastError());
     return 0;
