@@ -73,6 +73,7 @@ struct Geo {
     int ncell;
     int NJ;
     int nj[3];            // J accumulator nodes per axis: T + 1 + 2 jh
+    int cut;              // some tiles are shorter than T
     int jh;               // its halo (node layers beyond the tile on each side)
     int nmax;
     int s0;               // n[1] * n[2], row stride of x
@@ -874,10 +875,11 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     continue;
                 }
                 const bool active = lane < nruns;
-                int k = wave_incl_max(H[lane]), len = 0, pst = 0;  // the run's cell: c_cur + k
+                int k = wave_incl_max(H[lane]), len = 0, pst = 0, cell_runs = 0;  // the run's cell: c_cur + k
                 if (active) {
                     const int j = lane - R[k];
                     const int nr = R[k + 1] - R[k];
+                    cell_runs = nr;
                     const int p0 = (k == 0) ? pos_cur : s_seg[c_cur + k];
                     const int nc = s_seg[c_cur + k + 1] - p0;
                     const int bl = nc < (1 << 21) ? fdivi(nc, __builtin_amdgcn_rcpf((float)nr)) : nc / nr;
@@ -885,6 +887,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     len = bl + (j < rem ? 1 : 0);
                     pst = p0 + j * bl + min(j, rem);
                 }
+                const bool dense = __ballot(cell_runs > 3) != 0;
                 const int plo = __shfl(pst, 0, WS);
                 const int phi = __shfl(pst + len, nruns - 1, WS);
                 if (plo < 0 || (long long)phi > S.cap || phi - plo > WCH || phi < plo) {  // uniform over the wave
@@ -1195,12 +1198,14 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     }
                 if (MODE != MODE_REBIN && run_in > 0) {
                     if (!(jmax * (float)run_in <= g.fix_lim)) atomicOr(A.err, ERR_JSAT);
-                    // Lanes with runs of one cell start at different corners, corner q ^ (lane % 8): together
-                    // at the same one, their atomics on its node went one by one (push of 96^3 cells
-                    // with 300 a cell at the densest 1195 -> 982 us, 64^3 x 64 297 -> 277, 32^3 x 32 in
-                    // a reproducible order 64 -> 51.5, 8^3 x 512 72.5 -> 68; 128^3 x 32, four runs a
-                    // cell, 1045 either way).
-                    const bool fx = lane & 4, fy = lane & 2, fz = lane & 1;
+                    // Where a cell has more than three runs, lane l starts at corner l % 8 of its cell (corner
+                    // q ^ (l % 8) in turn q): together at the same one, the atomics of the cell's lanes on
+                    // that node went one by one (push of 96^3 cells with 300 a cell at the densest 1195 ->
+                    // 982 us, 64^3 x 64 297 -> 277, 32^3 x 32 in a reproducible order 64 -> 51.5, 8^3 x
+                    // 512 72.5 -> 68; 128^3 x 32, four runs a cell, 1045 either way, and 128^3 x 8, one
+                    // run, 370 without and 385).
+                    const int rot = dense ? lane : 0;
+                    const bool fx = rot & 4, fy = rot & 2, fz = rot & 1;
                     const int l0 = ((lx + JH + fx) * G.nj1 + (ly + JH + fy)) * G.nj2 + (lz + JH + fz);
                     const int dx = fx ? -G.nj1 * G.nj2 : G.nj1 * G.nj2, dy = fy ? -G.nj2 : G.nj2, dz = fz ? -1 : 1;
 #pragma unroll
@@ -1212,12 +1217,14 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                             N[q] = f ? b : a;
                             N[r] = f ? a : b;
                         };
+                        if (dense) {
 #pragma unroll
                         for (int q = 0; q < 4; ++q) swap_if(fx, q, q + 4);
 #pragma unroll
                         for (int q = 0; q < 4; ++q) swap_if(fy, (q & 2) * 2 + (q & 1), (q & 2) * 2 + (q & 1) + 2);
 #pragma unroll
                         for (int q = 0; q < 4; ++q) swap_if(fz, 2 * q, 2 * q + 1);
+                        }
 #pragma unroll
                         for (int q = 0; q < 8; ++q)
                             fix_add(&sJ[d * G.NJ + l0 + (q & 4 ? dx : 0) + (q & 2 ? dy : 0) + (q & 1 ? dz : 0)], N[q],
@@ -1366,8 +1373,14 @@ __device__ __forceinline__ float4 sum_partials(const FieldArgs& F, int i, int x,
                 const int tb = py[b] >> 8, lb = py[b] & 255;
                 const int tc = pz[cc] >> 8, lc = pz[cc] & 255;
                 const int tile = (ta * g.NTl[1] + tb) * g.NTl[2] + tc;
-                const TileBox bx = tile_at(g, ta, tb, tc);
-                const int h = 1 + 2 * g.jh, nj1 = bx.w1 + h, nj2 = bx.w2 + h, NJ = (bx.w0 + h) * nj1 * nj2;
+                int nj1 = g.nj[1], nj2 = g.nj[2], NJ = g.NJ;
+                if (g.cut) {
+                    const TileBox bx = tile_at(g, ta, tb, tc);
+                    const int h = 1 + 2 * g.jh;
+                    nj1 = bx.w1 + h;
+                    nj2 = bx.w2 + h;
+                    NJ = (bx.w0 + h) * nj1 * nj2;
+                }
                 const int l = (la * nj1 + lb) * nj2 + lc;
                 const float* base = F.jpart + (long long)tile * g.nsl * 3 * g.NJ;
 #pragma unroll 4
@@ -3234,6 +3247,7 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             g.sink_c[k] = (float)d.sink_center[k];
         }
         g.TC = g.T[0] * g.T[1] * g.T[2];
+        for (int k = 0; k < 3; ++k) g.cut |= g.n[k] % g.T[k] != 0;
         g.ntiles = g.NTl[0] * g.NTl[1] * g.NTl[2];
         {
             // One block per tile leaves most CUs idle on a grid of few tiles (8^3 cells: one tile).
