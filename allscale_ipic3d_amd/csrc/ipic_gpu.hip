@@ -2,8 +2,8 @@
 //
 // Device layout (one HIP stream per context):
 //   particles  per species, structure of arrays of FP32: cell-relative offsets ox,oy,oz (cell
-//              units) and velocities vx,vy,vz; 24 B per particle; sorted by cell in tile-major
-//              cell order (cid = tile * TC + local cell), ping-pong buffers X[0], X[1].
+//              units) and velocities vx,vy,vz; 24 B per particle; sorted by cell, the cells
+//              numbered tile by tile (TileBox), ping-pong buffers X[0], X[1].
 //   fields     E (nodes), Bc (centres), Bn (nodes), J (nodes) as float4 rows, row-major.
 //   J partials per tile and block slice: the tile's nodes plus IPIC_JHALO node layers on each
 //              side, (T+1+2h)^3 x 3 FP32, summed across tiles and slices in FP64 by the E pass.
@@ -1201,7 +1201,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     // Where a cell has more than three runs, lane l starts at corner l % 8 of its cell (corner
                     // q ^ (l % 8) in turn q): together at the same one, the atomics of the cell's lanes on
                     // that node went one by one (push of 96^3 cells with 300 a cell at the densest 1195 ->
-                    // 982 us, 64^3 x 64 297 -> 277, 32^3 x 32 in a reproducible order 64 -> 51.5, 8^3 x
+                    // 982 us, 64^3 x 64 297 -> 277, 32^3 x 64 in a reproducible order 64 -> 51.5, 8^3 x
                     // 512 72.5 -> 68; 128^3 x 32, four runs a cell, 1045 either way, and 128^3 x 8, one
                     // run, 370 without and 385).
                     const int rot = dense ? lane : 0;
