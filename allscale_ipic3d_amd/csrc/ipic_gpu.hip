@@ -1794,9 +1794,9 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int2* order, int ex
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int blocks = g.ntiles * g.nsl + extra;
     auto load = [&](int t) {
-        int v = 0;
+        long long v = 0;
         for (int sp = 0; sp < nsp; ++sp) v += A.sp[sp].tile_total[t];
-        return v;
+        return (int)min(v, 0x7fffffffll);  // (16 species may hold more)
     };
     // over the block: the sum of a, the maximum of m
     auto reduce = [&](unsigned long long& a, int& m) {
@@ -3247,6 +3247,7 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             g.sink_c[k] = (float)d.sink_center[k];
         }
         g.TC = g.T[0] * g.T[1] * g.T[2];
+        g.cut = 0;
         for (int k = 0; k < 3; ++k) g.cut |= g.n[k] % g.T[k] != 0;
         g.ntiles = g.NTl[0] * g.NTl[1] * g.NTl[2];
         {
