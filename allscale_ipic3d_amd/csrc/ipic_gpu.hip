@@ -1794,9 +1794,9 @@ __device__ void tile_order_block(const ScanArgs& A, int nsp, int2* order, int ex
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int blocks = g.ntiles * g.nsl + extra;
     auto load = [&](int t) {
-        long long v = 0;
+        int v = 0;  // (8 species of at most 178956970 particles: below 2^31)
         for (int sp = 0; sp < nsp; ++sp) v += A.sp[sp].tile_total[t];
-        return (int)min(v, 0x7fffffffll);  // (16 species may hold more)
+        return v;
     };
     // over the block: the sum of a, the maximum of m
     auto reduce = [&](unsigned long long& a, int& m) {
