@@ -2463,6 +2463,7 @@ struct ipic_ctx {
     bool j_summed = true;          // J holds the sum of the current tile partials (and overflow)
     bool canonical = true;
     bool track = false;
+    bool view_out = false;         // ipic_gpu_field_state gave out E and Bc: a caller may write them
     std::vector<void*> allocs;
     std::string err;
     hipEvent_t ev[8] = {};
@@ -2767,7 +2768,12 @@ int launch_leapfrog(ipic_ctx* ctx, bool node_b) {
     // the static field uses no J: it is formed on demand (download, conservation, field state)
     // from the current deposit, and the next deposit pass clears the overflow accumulator
     const int n = ctx->d.field_substeps;
-    if (n == 0) return 0;
+    if (n == 0) {
+        // its node B is what the upload formed, until a caller that was given Bc may have written it
+        // (the pass is 3 us at 8^3 cells; the dipole mover reads no node B)
+        const bool written = ctx->view_out && !(ctx->d.flags & IPIC_FLAG_DIPOLE_MOVER);
+        return node_b && written ? launch_c2n(ctx) : 0;
+    }
     if (n > 1) {
         // Two substeps a launch.  A launch swaps the buffers, and the arrays that ipic_gpu_field_state
         // hands out must stay the live ones: the number of launches is even, with 1 to 3 substeps
@@ -2950,7 +2956,6 @@ int field_phase(ipic_ctx* ctx, bool use_op, ipic_step_stats* st) {
         if (int rc = operator_phase(ctx, st)) return rc;
         if (int rc = launch_c2n(ctx)) return rc;
     } else {
-        // with interpC2N in its last launch; a static field keeps the node B that the upload formed
         if (int rc = launch_leapfrog(ctx, true)) return rc;
     }
     if (timing) {
@@ -3800,6 +3805,7 @@ int ipic_gpu_field_state(ipic_ctx* ctx, ipic_field_state* out) {
         if (int rc = launch_jsum(ctx)) return rc;
         if (work)
             if (int rc = wait_work(ctx)) return rc;
+        ctx->view_out = true;
         out->E = (float*)ctx->E;
         out->Bc = (float*)ctx->Bc;
         out->J = (float*)ctx->J;

@@ -211,7 +211,9 @@ typedef struct ipic_field_operator {
 int ipic_gpu_set_field_operator(ipic_ctx* ctx, const ipic_field_operator* op);
 
 /* Device view of the field state for a trainer (valid until the next call on ctx): float4
- * arrays of n^3 entries, (x, y, z, unused).  J is formed from the last deposit first. */
+ * arrays of n^3 entries, (x, y, z, unused).  J is formed from the last deposit first.  A
+ * caller may write Bc: the node B of the next step is formed from it, also with the static
+ * field. */
 typedef struct ipic_field_state {
     float* E;                     /* E - E0 on nodes */
     float* Bc;                    /* Bc - B0 on centres */
