@@ -54,6 +54,8 @@ def build(verbose: bool = False) -> list[str]:
 CPP_TESTS = {
     # C++ mirror of the reference's step API, driven by tests/test_cpp_mirror.py
     os.path.join(ROOT, "tests", "cpp", "ipic3d_mirror_test"): os.path.join(ROOT, "tests", "cpp", "ipic3d_mirror_test.cpp"),
+    # the library's host side over a stand-in for the HIP runtime, driven by tests/test_host_calls.py
+    os.path.join(ROOT, "tests", "cpp", "host_calls_test"): os.path.join(ROOT, "tests", "cpp", "host_calls_test.cpp"),
 }
 
 

@@ -2463,6 +2463,7 @@ struct ipic_ctx {
     bool j_summed = true;          // J holds the sum of the current tile partials (and overflow)
     bool canonical = true;
     bool track = false;
+    bool unfinished = false;       // a call failed and may have left work queued on the stream
     bool view_out = false;         // ipic_gpu_field_state gave out E and Bc: a caller may write them
     std::vector<void*> allocs;
     std::string err;
@@ -3164,15 +3165,18 @@ int check_ctx(ipic_ctx* ctx) {
 // instance) crosses the ABI; it becomes an error code with a message instead.
 template <class F>
 int guarded(ipic_ctx* ctx, F&& body) {
+    int rc = 0;
     try {
-        return body();
+        rc = body();
     } catch (const std::bad_alloc&) {
-        return fail(ctx, IPIC_E_RANGE, "out of host memory");
+        rc = fail(ctx, IPIC_E_RANGE, "out of host memory");
     } catch (const std::exception& e) {
-        return fail(ctx, IPIC_E_HIP, std::string("internal error: ") + e.what());
+        rc = fail(ctx, IPIC_E_HIP, std::string("internal error: ") + e.what());
     } catch (...) {
-        return fail(ctx, IPIC_E_HIP, "internal error");
+        rc = fail(ctx, IPIC_E_HIP, "internal error");
     }
+    if (rc && ctx) ctx->unfinished = true;
+    return rc;
 }
 
 }  // namespace
@@ -3797,14 +3801,17 @@ int ipic_gpu_field_state(ipic_ctx* ctx, ipic_field_state* out) {
     return guarded(ctx, [&]() -> int {
         if (int rc = check_ctx(ctx)) return rc;
         if (!out) return fail(ctx, IPIC_E_ARG, "null output");
-        const bool work = !ctx->j_valid || !ctx->j_summed;  // every call leaves the stream finished
+        // every call leaves the stream finished, unless it failed
+        const bool work = !ctx->j_valid || !ctx->j_summed || ctx->unfinished;
         if (!ctx->j_valid) {
             if (int rc = launch_particles(ctx, MODE_DEPOSIT)) return rc;
             ctx->j_valid = true;
         }
         if (int rc = launch_jsum(ctx)) return rc;
-        if (work)
+        if (work) {
             if (int rc = wait_work(ctx)) return rc;
+            ctx->unfinished = false;
+        }
         ctx->view_out = true;
         out->E = (float*)ctx->E;
         out->Bc = (float*)ctx->Bc;
