@@ -3312,11 +3312,15 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         }
         int rc = 0;
         const size_t nc = (size_t)g.ncell;
-        rc = rc ? rc : dalloc(ctx, &ctx->E, nc);
-        rc = rc ? rc : dalloc(ctx, &ctx->Bc, nc);
-        if (d.field_substeps > 1) {
-            rc = rc ? rc : dalloc(ctx, &ctx->E2, nc);
-            rc = rc ? rc : dalloc(ctx, &ctx->Bc2, nc);
+        // (with several substeps the second buffers lie behind the first: a context is created with as many
+        // allocations as without them)
+        const bool two = d.field_substeps > 1;
+        const size_t row = (nc + 15) / 16 * 16;  // the second starts on a cache line
+        rc = rc ? rc : dalloc(ctx, &ctx->E, two ? 2 * row : nc);
+        rc = rc ? rc : dalloc(ctx, &ctx->Bc, two ? 2 * row : nc);
+        if (!rc && two) {
+            ctx->E2 = ctx->E + row;
+            ctx->Bc2 = ctx->Bc + row;
         }
         rc = rc ? rc : dalloc(ctx, &ctx->Bn, nc);
         rc = rc ? rc : dalloc(ctx, &ctx->J, nc);
@@ -3350,11 +3354,13 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
         if (!rc)
             for (int k = 0; k < 8; ++k)
                 if (hipEventCreate(&ctx->ev[k]) != hipSuccess) rc = fail(ctx, IPIC_E_HIP, "hipEventCreate");
-        if (!rc && hipHostMalloc((void**)&ctx->hred, (size_t)ctx->red_blocks * 5 * sizeof(double)) != hipSuccess)
+        const size_t sums = (size_t)ctx->red_blocks * 5;  // 8-byte words, the report's behind them
+        if (!rc && hipHostMalloc((void**)&ctx->hred, (sums + REPORT_WORDS) * 8) != hipSuccess)
             rc = fail(ctx, IPIC_E_HIP, "hipHostMalloc");
-        if (!rc && hipHostMalloc((void**)&ctx->hrep, REPORT_WORDS * sizeof(unsigned long long)) != hipSuccess)
-            rc = fail(ctx, IPIC_E_HIP, "hipHostMalloc");
-        if (!rc) std::memset(ctx->hrep, 0, REPORT_WORDS * sizeof(unsigned long long));
+        if (!rc) {
+            ctx->hrep = (unsigned long long*)(ctx->hred + sums);
+            std::memset(ctx->hrep, 0, REPORT_WORDS * sizeof(unsigned long long));
+        }
         if (rc) {
             std::string msg = ctx->err;
             ipic_gpu_destroy(ctx);
@@ -3374,7 +3380,6 @@ int ipic_gpu_destroy(ipic_ctx* ctx) {
         for (int k = 0; k < 8; ++k)
             if (ctx->ev[k]) (void)hipEventDestroy(ctx->ev[k]);
         if (ctx->hred) (void)hipHostFree(ctx->hred);
-        if (ctx->hrep) (void)hipHostFree(ctx->hrep);
         if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return 0;

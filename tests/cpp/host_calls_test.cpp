@@ -1,9 +1,10 @@
 // Host-side checks of the library without a GPU: this program defines the HIP runtime calls that
 // libipic_gpu.so makes (its own definitions take precedence over the runtime's), runs no kernel,
-// notes what is queued, and can refuse a launch.
+// notes what is queued and allocated, and can refuse a launch.
 //
 //   host_calls_test --failed-step   after a step that fails with work queued, a call that hands out
 //                                   device pointers waits for that work
+//   host_calls_test --create        what creating a context allocates
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -12,7 +13,7 @@
 #include "ipic_gpu.h"
 
 namespace {
-int launches = 0, refuse = 0, error = 0;
+int launches = 0, refuse = 0, error = 0, device_allocs = 0, pinned_allocs = 0;
 bool queued = false;
 }  // namespace
 
@@ -20,9 +21,9 @@ extern "C" {
 struct Dim3 { unsigned x, y, z; };
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipDeviceGetAttribute(int* v, int, int) { *v = 256; return 0; }
-int hipMalloc(void** p, size_t n) { *p = std::calloc(1, n); return *p ? 0 : 2; }
+int hipMalloc(void** p, size_t n) { *p = std::calloc(1, n); ++device_allocs; return *p ? 0 : 2; }
 int hipFree(void* p) { std::free(p); return 0; }
-int hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(1, n); return *p ? 0 : 2; }
+int hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(1, n); ++pinned_allocs; return *p ? 0 : 2; }
 int hipHostFree(void* p) { std::free(p); return 0; }
 int hipMemcpy(void* d, const void* s, size_t n, int) { std::memcpy(d, s, n); return 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) { std::memcpy(d, s, n); queued = true; return 0; }
@@ -104,9 +105,25 @@ int failed_step() {
     return failed > 10 ? 0 : 1;
 }
 
+int create() {
+    int device[2];
+    for (int substeps : {1, 2}) {
+        device_allocs = pinned_allocs = 0;
+        ipic_gpu_destroy(make(substeps));
+        device[substeps - 1] = device_allocs;
+        if (pinned_allocs != 1) {
+            std::printf("%d pinned allocations\n", pinned_allocs);
+            return 1;
+        }
+    }
+    std::printf("%d and %d device allocations\n", device[0], device[1]);
+    return device[0] == device[1] ? 0 : 1;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc == 2 && !std::strcmp(argv[1], "--failed-step")) return failed_step();
+    if (argc == 2 && !std::strcmp(argv[1], "--create")) return create();
     return 2;
 }

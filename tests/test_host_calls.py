@@ -1,5 +1,5 @@
 """The library's host side without a GPU: tests/cpp/host_calls_test.cpp stands in for the HIP runtime,
-runs no kernel and notes what the library queues."""
+runs no kernel and notes what the library queues and allocates."""
 import os
 import subprocess
 
@@ -10,7 +10,7 @@ EXE = os.path.join(ROOT, "tests", "cpp", "host_calls_test")
 
 
 @pytest.mark.skipif(not os.path.exists(EXE), reason="host call test not built")
-@pytest.mark.parametrize("check", ["--failed-step"])
+@pytest.mark.parametrize("check", ["--failed-step", "--create"])
 def test_host_calls(check):
     r = subprocess.run([EXE, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
