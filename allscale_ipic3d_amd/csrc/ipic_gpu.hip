@@ -599,14 +599,14 @@ __device__ __forceinline__ void gather_regs(const float4 n4[8], const float2 n2[
     }
 }
 
-// Dynamic LDS layout of k_particles (bytes, 16-aligned sections)
+// Dynamic LDS layout of k_particles (bytes; the sections lie on multiples of what they hold)
 struct PLayout {
     int off_f4, off_f2, off_seg, off_cnt, off_wlo, off_wave, wave_bytes, total;
 };
 
-__host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF, bool track) {
-    PLayout L;
-    int o = 3 * NJ * 8;             // J, int64
+__host__ __device__ constexpr PLayout particle_layout(int NJ, int TC, int NF, bool track) {
+    PLayout L{};
+    int o = (3 * NJ * 8 + 15) & ~15;  // J, int64 (its nodes are an odd number in a tile of 8x8x8)
     L.off_f4 = o; o += NF * 16;     // node field (Ex,Ey,Ez,Bx)
     L.off_f2 = o; o += NF * 8;      // node field (By,Bz)
     L.off_seg = o; o += SPG * (TC + 1) * 4;  // segment starts of SPG species
@@ -622,6 +622,19 @@ __host__ __device__ inline PLayout particle_layout(int NJ, int TC, int NF, bool 
     L.total = o;
     return L;
 }
+
+constexpr bool layout_aligned() {
+    for (int a = 1; a <= 8; ++a)
+        for (int b = 1; b <= 8; ++b)
+            for (int c = 1; c <= 8; ++c)
+                for (int track = 0; track < 2; ++track) {
+                    const int h = 1 + 2 * IPIC_JHALO, NF = (a + 1) * (b + 1) * (c + 1);
+                    const PLayout L = particle_layout((a + h) * (b + h) * (c + h), a * b * c, NF, track != 0);
+                    if (L.off_f4 % 16 || L.off_f2 % 8 || L.off_seg % 4 || L.off_wave % 16 || L.wave_bytes % 16) return false;
+                }
+    return true;
+}
+static_assert(layout_aligned(), "float4 nodes on 16 bytes in every tile");
 
 __host__ __device__ inline int field_nodes(const Geo& g) { return (g.T[0] + 1) * (g.T[1] + 1) * (g.T[2] + 1); }
 
