@@ -515,8 +515,12 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float* part, int blocks
             const float4 p = s[k][c];
             v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
         }
+        // atomic: passes on several streams may add to one gradient
         float* g = grad + 4 * col;
-        g[0] += v.x; g[1] += v.y; g[2] += v.z; g[3] += v.w;
+        atomicAdd(g, v.x);
+        atomicAdd(g + 1, v.y);
+        atomicAdd(g + 2, v.z);
+        atomicAdd(g + 3, v.w);
     }
 }
 
