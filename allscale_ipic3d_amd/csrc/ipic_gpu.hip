@@ -36,23 +36,20 @@ namespace {
 #ifndef IPIC_PUSH_THREADS
 #define IPIC_PUSH_THREADS 256    // threads per block of the particle kernel
 #endif
-#ifndef IPIC_KRUN
-#define IPIC_KRUN 5              // max particles per run (one lane, held in registers)
-#endif
 #ifndef IPIC_JHALO
 #define IPIC_JHALO 0             // node layers of the tile J accumulator beyond the tile (0 or 1);
                                  // deposits beyond it go to the global overflow accumulator
 #endif
 #ifndef IPIC_PUSH_WAVES_PER_EU
 #define IPIC_PUSH_WAVES_PER_EU 3 // register budget of the particle kernel, waves per SIMD (0: the
-                                 // compiler's choice); see push_waves()
+                                 // compiler's choice)
 #endif
 
 constexpr int NT = 256;          // threads per block of the scan kernels
 constexpr int WS = 64;           // wavefront size
 constexpr int NTP = IPIC_PUSH_THREADS;
 constexpr int NW = NTP / WS;     // waves per block of the particle kernel
-constexpr int KRUN = IPIC_KRUN;
+constexpr int KRUN = 5;          // max particles per run (one lane, held in registers)
 constexpr int WCH = WS * KRUN;   // max particles per wave chunk
 constexpr int K0CAP = 32;        // leaver buffer entries per wave chunk
 constexpr int QCAP = 48;         // arrival queue entries per wave
@@ -543,10 +540,9 @@ __device__ __forceinline__ void stp(Rsrc r, float v, unsigned voff, unsigned sof
 }
 
 // v[0..3] to four consecutive floats in one dwordx4 store
-template <int N>
-__device__ __forceinline__ void st4(Rsrc r, unsigned voff, unsigned soff, const float (&v)[N]) {
+__device__ __forceinline__ void st4(Rsrc r, unsigned voff, unsigned soff, const float (&v)[KRUN]) {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const u4 q = {__float_as_uint(v[0]), __float_as_uint(v[1 % N]), __float_as_uint(v[2 % N]), __float_as_uint(v[3 % N])};
+    const u4 q = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
     __builtin_amdgcn_raw_buffer_store_b128(q, r, voff, soff, 0);
 }
 
@@ -643,10 +639,8 @@ enum { OPT_FIX8 = 1, OPT_SINK = 2, OPT_REFLECT = 4, OPT_DIPOLE = 8 };
 
 // Register budget (waves per SIMD) of a particle-kernel instance: every instance fits 168 VGPRs
 // (3 waves per SIMD) with runs of 5.
-constexpr int push_waves(bool, int) { return IPIC_PUSH_WAVES_PER_EU; }
-
 #if IPIC_PUSH_WAVES_PER_EU > 1
-#define IPIC_PUSH_ATTR __attribute__((amdgpu_waves_per_eu(push_waves(TRACK, OPT))))
+#define IPIC_PUSH_ATTR __attribute__((amdgpu_waves_per_eu(IPIC_PUSH_WAVES_PER_EU)))
 #else
 #define IPIC_PUSH_ATTR
 #endif
@@ -1032,7 +1026,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
 #pragma unroll
                 for (int m = 0; m < 8; ++m) mom[0][m] = mom[1][m] = mom[2][m] = 0.0f;
                 float jmax = 0.0f;  // largest |j| component of the run: bounds every corner sum / run_in
-                // this run's arrivals: particles that sit in another cell (queued by input index)
+                // this run's arrivals: particles that sit in another cell
                 unsigned amask = 0;
 #pragma unroll
                 for (int jj = 0; jj < KRUN; ++jj)
@@ -1119,7 +1113,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                     } else {
                         const unsigned vo = (unsigned)o0 * 4u;
                         // the first four of each array in one dwordx4 store, the rest one by one
-                        if (KRUN >= 4 && len >= 4) {
+                        if (len >= 4) {
                             st4(rout, vo, 0, rx);
                             st4(rout, vo, cs, ry);
                             st4(rout, vo, 2 * cs, rz);
@@ -1127,7 +1121,7 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                             st4(rout, vo, 4 * cs, rvy);
                             st4(rout, vo, 5 * cs, rvz);
                         }
-                        const int jlo = (KRUN >= 4 && len >= 4) ? 4 : 0;
+                        const int jlo = len >= 4 ? 4 : 0;
 #pragma unroll
                         for (int jj = 0; jj < KRUN; ++jj)
                             if (jj >= jlo && jj < len)
@@ -1232,11 +1226,11 @@ __global__ __launch_bounds__(NTP) IPIC_PUSH_ATTR void k_particles(PushArgs A) {
                         };
                         if (dense) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) swap_if(fx, q, q + 4);
+                            for (int q = 0; q < 4; ++q) swap_if(fx, q, q + 4);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) swap_if(fy, (q & 2) * 2 + (q & 1), (q & 2) * 2 + (q & 1) + 2);
+                            for (int q = 0; q < 4; ++q) swap_if(fy, (q & 2) * 2 + (q & 1), (q & 2) * 2 + (q & 1) + 2);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) swap_if(fz, 2 * q, 2 * q + 1);
+                            for (int q = 0; q < 4; ++q) swap_if(fz, 2 * q, 2 * q + 1);
                         }
 #pragma unroll
                         for (int q = 0; q < 8; ++q)
@@ -2775,7 +2769,6 @@ void launch_leap(ipic_ctx* ctx, int last) {
 }
 
 int launch_c2n(ipic_ctx* ctx);
-int launch_jsum(ipic_ctx* ctx);
 
 // The field substeps with J held fixed, and with node_b the gather's node B.
 int launch_leapfrog(ipic_ctx* ctx, bool node_b) {
