@@ -595,7 +595,9 @@ __device__ __forceinline__ void gather_regs(const float4 n4[8], const float2 n2[
     }
 }
 
-// Dynamic LDS layout of k_particles (bytes; the sections lie on multiples of what they hold)
+// Dynamic LDS layout of k_particles (bytes; the sections lie on multiples of what they hold: with the
+// float4 nodes 8 bytes off, 128^3 x 32 waited eight times as long on LDS, SQ_WAIT_INST_LDS 4.3e7
+// against 5.7e6, and four steps took 4921 us against 4877)
 struct PLayout {
     int off_f4, off_f2, off_seg, off_cnt, off_wlo, off_wave, wave_bytes, total;
 };
@@ -3342,15 +3344,23 @@ int ipic_gpu_create(const ipic_desc* desc, ipic_ctx** out) {
             Species& S = ctx->sp[s];
             S.q = d.species[s].q;
             S.qom = d.species[s].qom;
-            rc = rc ? rc : dalloc(ctx, &S.seg, nc + 1);
-            rc = rc ? rc : dalloc(ctx, &S.start, nc + 1);
-            rc = rc ? rc : dalloc(ctx, &S.stay, nc);
-            rc = rc ? rc : dalloc(ctx, &S.cnt_acc, nc);
-            rc = rc ? rc : dalloc(ctx, &S.stay_acc, nc);
-            rc = rc ? rc : dalloc(ctx, &S.arr, nc);
-            rc = rc ? rc : dalloc(ctx, &S.tile_total, (size_t)g.ntiles);
-            rc = rc ? rc : dalloc(ctx, &S.group_total, ((size_t)g.ntiles + NT - 1) / NT);
-            if (d.flags & IPIC_FLAG_REPRODUCIBLE) rc = rc ? rc : dalloc(ctx, &S.work, nc + 1);
+            // one allocation for the species' per-cell and per-tile arrays: two species at 8^3 are created in
+            // 140 us instead of 205, at 32^3 in 180 instead of 245
+            const size_t tiles = (size_t)g.ntiles, work = (d.flags & IPIC_FLAG_REPRODUCIBLE) ? nc + 1 : 0;
+            const struct { int** p; size_t n; } parts[] = {
+                {&S.seg, nc + 1}, {&S.start, nc + 1}, {&S.stay, nc},          {&S.cnt_acc, nc},
+                {&S.stay_acc, nc}, {&S.arr, nc},      {&S.tile_total, tiles}, {&S.group_total, (tiles + NT - 1) / NT},
+                {&S.work, work}};
+            auto padded = [](size_t n) { return (n + 63) / 64 * 64; };  // each starts on 256 bytes
+            size_t all = 0;
+            for (const auto& q : parts) all += padded(q.n);
+            int* base = nullptr;
+            rc = dalloc(ctx, &base, all);
+            for (const auto& q : parts) {
+                if (rc || q.n == 0) continue;
+                *q.p = base;
+                base += padded(q.n);
+            }
         }
         if (!rc) {
             e = hipMemcpyAsync(ctx->jpairs, jp.data(), jp.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream);
