@@ -6,13 +6,15 @@
 // Activations are channel-last on the n^3 index lattice: X[v * C + c], v = (x * ny + y) * nz + z.
 //
 // Forward convolution (k_conv): one persistent block per CU stages the layer's weights in LDS
-// once and walks a contiguous range of 4x4x16 (or 4x2x16) bricks of output voxels, two at a time,
-// computing every output channel of a brick.  The brick's input halo (6x6x18 voxels x CIN
-// channels) is staged in LDS, its 16-byte pieces permuted so that operand reads are
-// conflict-free, and the next brick's halo is loaded into registers while the current brick
-// computes.  Each wave owns one x-plane of the brick, i.e. four 16-voxel z-rows, and for every tap
-// issues one MFMA per (row, 16-output-channel tile): the A operand is 16 output x 32 (or 16) input
-// channels of the tap's weights, the B operand the input channels of 16 voxels, both from LDS.
+// once and walks a contiguous range of bricks of output voxels, two at a time, computing every
+// output channel of a brick.  A brick is 4 x R x 16 voxels with R = 1 to 5 rows (the rule stands at
+// conv(); the last brick of a column may be shorter).  Its input halo (6 x R+2 x 18 voxels x CIN
+// channels) is staged in LDS, its 16-byte pieces permuted (swz).  Up to 4 rows the next brick's halo is
+// loaded into registers while the current brick computes; 5 rows leave no registers for it, and it
+// is requested after the epilogue.  Each wave owns one x-plane of the brick, i.e. R 16-voxel z-rows, and
+// for every tap issues one MFMA per (row, 16-output-channel tile): the A operand is 16 output x 32
+// (or 16) input channels of the tap's weights, the B operand the input channels of 16 voxels, both
+// from LDS.
 // A lane then holds 4 consecutive output channels of a voxel.  The epilogue adds the bias,
 // optionally multiplies by silu'(z_saved) and adds a residual, and writes FP32 and/or BF16
 // (optionally silu-activated) outputs, 16 bytes a lane.
@@ -144,8 +146,10 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a, int nbricks) {
     const int m = lane & 15, kq = lane >> 4;
     unsigned char* hx_ = sx[half];
 
-    // 16-byte piece p of row r lies at piece p ^ swz(r): the 16 lanes that read one piece of 16
-    // consecutive rows then touch every bank once
+    // 16-byte piece p of row r lies at piece p ^ swz(r), so that one piece of 16 consecutive rows covers
+    // every bank once.  Not free of conflicts by the counters: 3.5 conflict cycles an LDS instruction at
+    // 64^3, 32 to 32 channels (0.8 with 8-byte padded rows, which need two reads an operand); LDS is
+    // active a quarter of the time.
     auto swz = [](int r) { return CIN == 32 ? (r >> 2) & 3 : (r >> 3) & 1; };
 
     // the next brick's halo travels in registers while the current brick computes: this thread
