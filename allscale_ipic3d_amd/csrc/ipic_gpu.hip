@@ -2178,7 +2178,7 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(256) void k_init(Geo g, const int* start, float* X, uint32_t* ids, long long cap,
+__global__ __launch_bounds__(256) void k_init(Geo g, const int* start, const int* id0, float* X, uint32_t* ids, long long cap,
                                               long long total, uint64_t seed, int species, double vx_, double vy_,
                                               double vz_, double dx_, double dy_, double dz_) {
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2208,7 +2208,7 @@ __global__ __launch_bounds__(256) void k_init(Geo g, const int* start, float* X,
     X[3 * cap + p] = (float)(dx_ + vx_ * n0);
     X[4 * cap + p] = (float)(dy_ + vy_ * n1);
     X[5 * cap + p] = (float)(dz_ + vz_ * n2);
-    if (ids) ids[p] = (uint32_t)p;
+    if (ids) ids[p] = (uint32_t)(id0[cid] + idx);
 }
 
 __device__ __forceinline__ double block_sum_d(double v, double* s) {
@@ -3543,11 +3543,37 @@ int ipic_gpu_init_particles(ipic_ctx* ctx, int32_t species, const int32_t* ppc, 
         Species& S = ctx->sp[species];
         if (int rc = set_layout(ctx, species, start)) return rc;
         if (total > 0) {
+            // Ids count the particles through the cells of tiles that divide the grid (the given ones, else the
+            // largest edge up to 8), whatever tiles the context works with.
+            const int* id0 = S.start;
+            Geo h = g;
+            for (int k = 0; k < 3 && ctx->track; ++k) {
+                int T = ctx->d.tile[k] > 0 ? ctx->d.tile[k] : std::min(g.n[k], 8);
+                while (g.n[k] % T != 0) --T;
+                h.T[k] = T;
+                h.NTl[k] = g.n[k] / T;
+            }
+            const bool renumber = h.T[0] != g.T[0] || h.T[1] != g.T[1] || h.T[2] != g.T[2];
+            std::vector<int> first(renumber ? nc : 0);
+            if (renumber) {
+                int at = 0;
+                for (int c = 0; c < nc; ++c) {
+                    int x, y, z;
+                    cell_of(h, c, x, y, z);
+                    const int cid = host_cid(g, x, y, z);
+                    first[cid] = at;
+                    at += start[cid + 1] - start[cid];
+                }
+                // they pass through an accumulator, which is zero before and after
+                HIPCK(ctx, hipMemcpyAsync(S.stay_acc, first.data(), nc * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+                id0 = S.stay_acc;
+            }
             const unsigned nb = (unsigned)((total + 255) / 256);
-            hipLaunchKernelGGL(k_init, dim3(nb), dim3(256), 0, ctx->stream, g, S.start, S.X[S.cur],
+            hipLaunchKernelGGL(k_init, dim3(nb), dim3(256), 0, ctx->stream, g, S.start, id0, S.X[S.cur],
                                ctx->track ? S.ids[S.cur] : nullptr, S.cap, total, seed, (int)species, vth[0], vth[1], vth[2],
                                drift[0], drift[1], drift[2]);
             HIPCK(ctx, hipGetLastError());
+            if (renumber) HIPCK(ctx, hipMemsetAsync(S.stay_acc, 0, nc * sizeof(int), ctx->stream));
         }
         HIPCK(ctx, hipStreamSynchronize(ctx->stream));
         ctx->j_valid = false;
